@@ -144,6 +144,13 @@ __device__ __forceinline__ uint32_t pick_halves(uint32_t a, int ia, uint32_t b, 
   return __builtin_amdgcn_perm(a, b, sel_lo | (sel_hi << 16));
 }
 
+// LDS transpose read: the 16 lanes of a group read 16 x 16-bit rows of 4 keys and each gets 4 consecutive
+// keys of one dim.
+__device__ __forceinline__ u32x2 ld_tr(const char* p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
+}
+
 // ---------------------------------------------------------------- global -> LDS DMA and its waits
 
 __device__ __forceinline__ unsigned lds_offset(const void* p) {

@@ -130,11 +130,6 @@ __device__ __forceinline__ void stage_store(u32x4 x, int w, int lane, char* slot
 
 // ---------------------------------------------------------------- MFMA operands from LDS
 
-__device__ __forceinline__ u32x2 ld_tr(const char* p) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
-}
-
 struct STile {
   f32x16 s[2];  // s[b][r]: key 32 b + 8 (r / 4) + 4 h + r % 4 of the tile, row n
 };

@@ -1,0 +1,81 @@
+"""The bf16 / fp16 matrix-core kernels behind `prefill` (Dh 64 and 128) at the sizes where they can go wrong:
+edges of the 32- and 64-key tiles and of the 32- and 128-row workgroups, one query on a long context, every
+group size, padding masks (whole padded tiles, windows past 4,096 keys, rows without a real key), unaligned
+views, and values that are not finite behind masked keys.  Against the oracle in float64."""
+
+import pytest
+import torch
+
+from oracle import torch_ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _inputs(b, h, hkv, tq, tk, dh, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(b, t, n, dh, generator=g).to(dtype).transpose(1, 2)
+            for t, n in ((tq, h), (tk, hkv), (tk, hkv))]
+
+
+def _run(q, k, v, key_valid=None):
+    from minillm.attention import get_backend
+
+    to = lambda x: x.transpose(1, 2).to(DEV).transpose(1, 2)  # noqa: E731  (keeps the [B, T, H, Dh] storage)
+    return get_backend("hip").prefill(to(q), to(k), to(v), key_valid=None if key_valid is None else key_valid.to(DEV)).cpu()
+
+
+def _compare(out, ref, dtype):
+    # the output's own rounding (2^-9 bf16, 2^-12 fp16 of the value, doubled), plus the weights' 16 bits or more:
+    # 2^-16 of |v| <= 6, and fp32 sums: 2e-4 covers both
+    torch.testing.assert_close(out.double(), ref, rtol=2 ** (-8 if dtype == torch.bfloat16 else -11), atol=2e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,h,hkv,tq,tk,dh", [
+    (1, 4, 4, 1, 1, 128), (2, 8, 2, 31, 31, 64), (1, 8, 2, 33, 65, 128), (1, 32, 8, 1, 1000, 128), (3, 4, 4, 5, 129, 64),
+    (1, 8, 1, 63, 64, 128), (1, 32, 1, 3, 97, 128), (2, 12, 4, 40, 71, 64), (2, 64, 64, 520, 520, 128),
+    (3, 96, 32, 257, 384, 64), (1, 128, 8, 511, 701, 128)])
+def test_edges(hip, dtype, b, h, hkv, tq, tk, dh):
+    q, k, v = _inputs(b, h, hkv, tq, tk, dh, dtype)
+    _compare(_run(q, k, v), torch_ref.prefill(q.double(), k.double(), v.double()), dtype)
+
+
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("b,h,hkv,tq,tk", [(3, 8, 2, 70, 200), (4, 64, 64, 300, 333), (2, 2, 1, 3, 4700)])
+def test_key_valid(hip, dh, b, h, hkv, tq, tk):
+    q, k, v = _inputs(b, h, hkv, tq, tk, dh, torch.bfloat16, seed=1)
+    valid = torch.rand(b, tk, generator=torch.Generator().manual_seed(2)) < 0.7
+    valid[0, :tk - tq // 2] = False  # the first queries of row 0 have no real key
+    valid[1] = torch.arange(tk) >= tk // 2  # left padding of whole tiles
+    if b > 2:
+        valid[2] = False  # no real key at all
+    _compare(_run(q, k, v, valid), torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid), torch.bfloat16)
+
+
+@pytest.mark.parametrize("h", [2, 128])
+def test_values_behind_masked_keys_do_not_leak(hip, h):
+    # key 40 is not finite: queries before it and (masked) all queries of batch row 1 never see it
+    b, t = 2, 300
+    q, k, v = _inputs(b, h, h, t, t, 128, torch.bfloat16, seed=3)
+    valid = torch.ones(b, t, dtype=torch.bool)
+    valid[1, 40] = False
+    ref = torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid)
+    for bad in (float("nan"), float("inf")):
+        v2 = v.clone()
+        v2[:, :, 40, 7] = bad
+        out = _run(q, k, v2, valid)
+        _compare(out[0, :, :40], ref[0, :, :40], torch.bfloat16)
+        _compare(out[1], ref[1], torch.bfloat16)
+        seen = out[0, :, 40:, 7].float()
+        assert (torch.isnan(seen) if bad != bad else seen == bad).all()
+        _compare(out[0, :, 40:, 8:], ref[0, :, 40:, 8:], torch.bfloat16)
+
+
+def test_unaligned_rows_and_large_scores(hip):
+    q, k, v = _inputs(1, 4, 2, 50, 80, 64, torch.float16, seed=4)
+    wide = torch.zeros(1, 4, 50, 65, dtype=torch.float16)
+    wide[..., 1:] = q
+    _compare(_run(wide[..., 1:], k, v), torch_ref.prefill(q.double(), k.double(), v.double()), torch.float16)
+    q, k = q * 30, k * 30  # scores of some thousands: one key takes all the weight, the max moves far
+    _compare(_run(q, k, v), torch_ref.prefill(q.double(), k.double(), v.double()), torch.float16)
