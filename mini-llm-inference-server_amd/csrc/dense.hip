@@ -8,9 +8,10 @@
 //                       four wavefronts share each 64-key K/V tile through LDS (many rows);
 //   dense_split_kernel  the same operands: workgroups of 32 query rows whose four wavefronts share the keys
 //                       out among them and merge their partial results in LDS (few rows);
-//   dense_kernel        everything else (any Dh up to 256, any strides, fp32), one workgroup per query row,
-//                       fp32 scalar arithmetic.
-// Scores and the running max and sum are fp32 everywhere.  The MFMA kernels give the PV product the fp32
+//   dense_f32_kernel    fp32, Dh 64 or 128, 16-byte aligned rows, on the fp32 MFMA instructions;
+//   dense_kernel        everything else (any Dh up to 256, any strides), one workgroup per query row, fp32 scalar
+//                       arithmetic.
+// Scores and the running max and sum are fp32 everywhere.  The 16-bit MFMA kernels give the PV product the fp32
 // probabilities as two 16-bit operands, P = hi + lo (lo = the rounding error of hi), so that a weight keeps
 // 16 significant bits or more instead of the 8 of a bf16 P.
 #include <math.h>
@@ -274,7 +275,8 @@ __device__ __forceinline__ void row_by_key(const DenseArgs& a, int b, int h, int
     float s = -INFINITY;
     if (allowed) {
       float dot = 0.f;
-      for (int d = 0; d < a.Dh; ++d) dot += ld_elem<DT>(a.q, q_row + d) * ld_elem<DT>(a.k, k_row0 + (int64_t)j * a.k_st + d);
+      const int64_t kr = k_row0 + (int64_t)j * a.k_st;
+      for (int d = 0; d < a.Dh; ++d) dot += ld_elem<DT>(a.q, q_row + d) * ld_elem<DT>(a.k, kr + d);
       s = dot * a.scale;
     }
     float cm = s;
@@ -773,13 +775,197 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// What the MFMA kernels take besides the head size: 16-byte aligned rows, key rows at most 32 MB apart (32-bit
-// offsets within a tile), a positive scale (the running max is kept in unscaled scores).
-bool mfma_operands(const DenseArgs& a) {
+// ---------------------------------------------------------------- fp32 on the matrix cores
+// 16 query rows (row = token * G + head) per workgroup of four wavefronts; wavefront w takes the 16-key tiles w, w + 4,
+// .. straight from global memory into registers, and the four partial (m, l, O) of each row are merged in LDS.
+//   S^T[16 keys x 16 rows] = K . Q^T     DH / 4 x v_mfma_f32_16x16x4_f32: lane (n, g) holds K row n and Q row n at
+//                                        dims 16 j + 4 g .. +3 (16-byte loads), product (j, e) takes element e, so the
+//                                        dims run through k in that order on both sides
+//   O^T[Dh x 16 rows]     += V^T . P^T   DH / 4 products: key step i takes the keys 4 g + i, whose P is register i of
+//                                        S^T's lane; lane (n, g) holds V row 4 g + i at dims 64 x + 4 n .. +3, so
+//                                        product (x, e)'s row r is dim 64 x + 4 r + e
+// Bound by the fp32 MFMA stream (64 x 32 cycles a tile) and the softmax between its halves.  One workgroup per
+// query row on the vector ALU took 316.4 us for 300 queries on 700 keys (8 query, 2 KV heads, Dh 128), this kernel
+// 21.2 us with four wavefronts (eight: 22.9, two: 37.3 us; four sequences of 550 tokens with 32 and 8 heads: 138 us
+// with four, 210 with eight, 128 with two), at 3.2e-7 from float64 against 4.7e-7.  Loading the next tile into a
+// second register set measured no faster.
+// Everything stays fp32 (the products of v_mfma_f32 are fp32 fused multiply-adds) with expf, and the running max moves
+// on every tile.
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ float max_xor16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+constexpr int kWavesF32 = 4;
+template <int DH, bool MASKED>
+__global__ __launch_bounds__(64 * kWavesF32) void dense_f32_kernel(const DenseArgs a) {
+  constexpr int W = kWavesF32, kBN = 16, kJ = DH / 16, kX = DH / 64;
+  constexpr int kPad = DH + 4;  // floats per row of the merge buffer: rows 16 bytes apart in the banks
+  __shared__ __attribute__((aligned(16))) float part[W][16][kPad];
+  __shared__ float2 ml[W][16];
+  __shared__ uint32_t bad_rows;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tokens = 16 / a.G;
+  const Item it = item_of(a, tokens);
+  const int off = a.Tk - a.Tq;
+  const int tok = it.t0 + n / a.G;
+  const bool row_valid = tok < a.Tq;
+  const int head = it.kvh * a.G + n % a.G;
+  const int qp = row_valid ? off + tok : a.Tk - 1;
+  const int qp_lo = off + it.t0;
+  const int kv_end = off + min(it.t0 + tokens, a.Tq), last = kv_end - 1;
+  const int ntiles = (kv_end + kBN - 1) / kBN;
+  if (threadIdx.x == 0) bad_rows = 0;
+
+  KeyMask km;
+  int ts = 0;
+  if constexpr (MASKED) {
+    find_first(a, it.b, kv_end, lane, km);
+    ts = min(km.first, qp_lo) / kBN;
+    if (ts / 4 / 64 * 64 != km.base) load_window(a, it.b, ts / 4 / 64 * 64, lane, km);
+  }
+
+  const int kvh = it.kvh * a.G / (a.H / a.Hkv);
+  const float* kc = reinterpret_cast<const float*>(a.k) + (int64_t)it.b * a.k_sb + (int64_t)kvh * a.k_sh;
+  const float* vc = reinterpret_cast<const float*>(a.v) + (int64_t)it.b * a.v_sb + (int64_t)kvh * a.v_sh;
+  f32x4 kf[kJ], vf[4][kX], qf[kJ];
+  auto load_k = [&](int t) {
+    const float* p = kc + (int64_t)min(t * kBN + n, last) * a.k_st + 4 * g;
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) kf[j] = *reinterpret_cast<const f32x4*>(p + 16 * j);
+  };
+  auto load_v = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* p = vc + (int64_t)min(t * kBN + 4 * g + i, last) * a.v_st + 4 * n;
+#pragma unroll
+      for (int x = 0; x < kX; ++x) vf[i][x] = *reinterpret_cast<const f32x4*>(p + 64 * x);
+    }
+  };
+  int t = ts + wave;
+  load_k(t);
+  load_v(t);
+  {
+    const float* q = reinterpret_cast<const float*>(a.q) + (int64_t)it.b * a.q_sb + (int64_t)head * a.q_sh +
+                     (int64_t)(row_valid ? tok : 0) * a.q_st + 4 * g;
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) {
+      qf[j] = *reinterpret_cast<const f32x4*>(q + 16 * j);
+      if (!row_valid) qf[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  f32x4 o[kX][4];
+#pragma unroll
+  for (int x = 0; x < kX; ++x)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[x][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  for (; t < ntiles; t += W) {
+    f32x4 s2[2] = {};  // two chains
+#pragma unroll
+    for (int j = 0; j < kJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s2[e & 1] = mfma_f32(kf[j][e], qf[j][e], s2[e & 1]);
+    load_k(t + W);  // past the last tile: copies of the last row, unused
+    f32x4 s = (s2[0] + s2[1]) * a.scale;
+    const int key0 = t * kBN + 4 * g;
+    uint32_t vm = 0xffffu;
+    if constexpr (MASKED) {
+      if (t / 4 - km.base >= 64) load_window(a, it.b, t / 4, lane, km);
+      vm = (uint32_t)(mask_word(km, t / 4) >> (16 * (t & 3))) & 0xffffu;
+    }
+    if (MASKED && vm != 0xffffu) {
+      const bool own = qp < km.first;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool see = own ? key0 + i == qp : (((vm >> (4 * g + i)) & 1u) != 0 && key0 + i <= qp);
+        s[i] = see ? s[i] : -INFINITY;
+      }
+    } else if (t * kBN + kBN - 1 > qp_lo) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[i] = key0 + i > qp ? -INFINITY : s[i];
+    }
+    const float mx = max_xor32(max_xor16(__builtin_fmaxf(__builtin_fmaxf(s[0], s[1]), __builtin_fmaxf(s[2], s[3]))));
+    const float m_new = fmaxf(m_run, mx);
+    const float alpha = m_new == m_run ? 1.f : expf(m_run - m_new);
+    float p[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = s[i] == -INFINITY ? 0.f : expf(s[i] - m_new);
+    l_run = l_run * alpha + sum_xor32(sum_xor16((p[0] + p[1]) + (p[2] + p[3])));
+    m_run = m_new;
+#pragma unroll
+    for (int x = 0; x < kX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[x][e] *= alpha;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int x = 0; x < kX; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[x][e] = mfma_f32(vf[i][x][e], p[i], o[x][e]);
+    load_v(t + W);
+  }
+
+  // o[x][e][r] is dim 64 x + 16 g + 4 r + e of row n
+#pragma unroll
+  for (int x = 0; x < kX; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<f32x4*>(&part[wave][n][64 * x + 16 * g + 4 * r]) =
+          f32x4{o[x][0][r], o[x][1][r], o[x][2][r], o[x][3][r]};
+  if (g == 0) ml[wave][n] = make_float2(m_run, l_run);
+  __syncthreads();
+  constexpr int kVecs = 16 * DH / 4, kPer = (kVecs + 64 * W - 1) / (64 * W);  // 16-byte pieces of the output, per thread
+  f32x4 res[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int idx = u * 64 * W + (int)threadIdx.x, row = idx / (DH / 4), d = 4 * (idx % (DH / 4));
+    if (idx < kVecs) {
+      float m = -INFINITY, l = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) m = fmaxf(m, ml[w][row].x);
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const float2 y = ml[w][row];
+        const float wgt = y.x == m ? 1.f : expf(y.x - m);  // a wavefront without a key of this row: 0
+        l += wgt * y.y;
+        v += wgt * *reinterpret_cast<const f32x4*>(&part[w][row][d]);
+      }
+      res[u] = v / l;
+      const f32x4 z = res[u];
+      if (z[0] != z[0] || z[1] != z[1] || z[2] != z[2] || z[3] != z[3]) atomicOr(&bad_rows, 1u << row);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int idx = u * 64 * W + (int)threadIdx.x, row = idx / (DH / 4), d = 4 * (idx % (DH / 4));
+    const int rtok = it.t0 + row / a.G;
+    if (idx < kVecs && rtok < a.Tq && !((bad_rows >> row) & 1u))
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + (int64_t)it.b * a.o_sb +
+                                (int64_t)(it.kvh * a.G + row % a.G) * a.o_sh + (int64_t)rtok * a.o_st + d) = res[u];
+  }
+  for (uint32_t bad = bad_rows; bad; bad &= bad - 1) {
+    const int row = __builtin_ctz(bad);
+    const int rtok = it.t0 + row / a.G;
+    if (row % W == wave && rtok < a.Tq)
+      row_by_key<MLLM_DTYPE_F32>(a, it.b, it.kvh * a.G + row % a.G, rtok, km.first, lane);
+  }
+}
+
+// What the MFMA kernels take besides the head size: 16-byte aligned rows (per16 elements in 16 bytes), key rows at
+// most 32 MB apart (32-bit offsets within a tile), a positive scale (the running max is kept in unscaled scores).
+bool mfma_operands(const DenseArgs& a, int per16) {
   const uintptr_t ptrs = (uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out;
   const int64_t strides = a.q_sb | a.q_sh | a.q_st | a.k_sb | a.k_sh | a.k_st | a.v_sb | a.v_sh | a.v_st | a.o_sb |
                           a.o_sh | a.o_st;
-  return ptrs % 16 == 0 && strides % 8 == 0 && a.k_st >= 0 && a.v_st >= 0 && a.k_st < (1 << 24) &&
+  return ptrs % 16 == 0 && strides % per16 == 0 && a.k_st >= 0 && a.v_st >= 0 && a.k_st < (1 << 24) &&
          a.v_st < (1 << 24) && a.scale > 0.f && a.scale < INFINITY && a.Tk < (1 << 30);
 }
 
@@ -811,6 +997,23 @@ int launch_mfma(const DenseArgs& a, hipStream_t st) {
   return check_launch("mllm_dense_attention");
 }
 
+int launch_f32(const DenseArgs& a, hipStream_t st) {
+  const int tokens = 16 / a.G;
+  const int64_t items = (int64_t)((a.Tq + tokens - 1) / tokens) * a.B * (a.H / a.G);
+  MLLM_REQUIRE(items < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_dense_attention: grid too large");
+  if (a.Dh == 128) {
+    if (a.key_valid)
+      dense_f32_kernel<128, true><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+    else
+      dense_f32_kernel<128, false><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+  } else if (a.key_valid) {
+    dense_f32_kernel<64, true><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+  } else {
+    dense_f32_kernel<64, false><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+  }
+  return check_launch("mllm_dense_attention");
+}
+
 }  // namespace
 }  // namespace mllm
 
@@ -837,7 +1040,11 @@ extern "C" int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, i
               kv_len, head_dim, pack, softmax_scale};
   dim3 grid(q_len, num_heads, batch);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype != MLLM_DTYPE_F32 && mfma_operands(a)) {
+  if (dtype == MLLM_DTYPE_F32 && (head_dim == 128 || head_dim == 64) && mfma_operands(a, 4)) {
+    a.G = 16 % group == 0 ? group : 1;
+    return launch_f32(a, st);
+  }
+  if (dtype != MLLM_DTYPE_F32 && mfma_operands(a, 8)) {
     const bool bf16 = dtype == MLLM_DTYPE_BF16;
     if (head_dim == 128)
       return bf16 ? launch_mfma<BF16, 128>(a, st) : launch_mfma<F16, 128>(a, st);

@@ -1,5 +1,5 @@
-"""The bf16 / fp16 matrix-core kernels behind `prefill` (Dh 64 and 128) at the sizes where they can go wrong:
-edges of the 32- and 64-key tiles and of the 32- and 128-row workgroups, one query on a long context, every
+"""The matrix-core kernels behind `prefill` (Dh 64 and 128) at the sizes where they can go wrong:
+edges of the 16-, 32- and 64-key tiles and of the 16-, 32- and 128-row workgroups, one query on a long context, every
 group size, padding masks (whole padded tiles, windows past 4,096 keys, rows without a real key), unaligned
 views, and values that are not finite behind masked keys.  Against the oracle in float64."""
 
@@ -26,12 +26,15 @@ def _run(q, k, v, key_valid=None):
 
 
 def _compare(out, ref, dtype):
+    if dtype == torch.float32:  # sums of up to 1,000 terms: a few times 2^-24 of the terms' size
+        torch.testing.assert_close(out.double(), ref, rtol=1e-5, atol=1e-5)
+        return
     # the output's own rounding (2^-9 bf16, 2^-12 fp16 of the value, doubled), plus the weights' 16 bits or more:
     # 2^-16 of |v| <= 6, and fp32 sums: 2e-4 covers both
     torch.testing.assert_close(out.double(), ref, rtol=2 ** (-8 if dtype == torch.bfloat16 else -11), atol=2e-4)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("b,h,hkv,tq,tk,dh", [
     (1, 4, 4, 1, 1, 128), (2, 8, 2, 31, 31, 64), (1, 8, 2, 33, 65, 128), (1, 32, 8, 1, 1000, 128), (3, 4, 4, 5, 129, 64),
     (1, 8, 1, 63, 64, 128), (1, 32, 1, 3, 97, 128), (2, 12, 4, 40, 71, 64), (2, 64, 64, 520, 520, 128),
@@ -41,23 +44,25 @@ def test_edges(hip, dtype, b, h, hkv, tq, tk, dh):
     _compare(_run(q, k, v), torch_ref.prefill(q.double(), k.double(), v.double()), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("b,h,hkv,tq,tk", [(3, 8, 2, 70, 200), (4, 64, 64, 300, 333), (2, 2, 1, 3, 4700)])
-def test_key_valid(hip, dh, b, h, hkv, tq, tk):
-    q, k, v = _inputs(b, h, hkv, tq, tk, dh, torch.bfloat16, seed=1)
+def test_key_valid(hip, dtype, dh, b, h, hkv, tq, tk):
+    q, k, v = _inputs(b, h, hkv, tq, tk, dh, dtype, seed=1)
     valid = torch.rand(b, tk, generator=torch.Generator().manual_seed(2)) < 0.7
     valid[0, :tk - tq // 2] = False  # the first queries of row 0 have no real key
     valid[1] = torch.arange(tk) >= tk // 2  # left padding of whole tiles
     if b > 2:
         valid[2] = False  # no real key at all
-    _compare(_run(q, k, v, valid), torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid), torch.bfloat16)
+    _compare(_run(q, k, v, valid), torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("h", [2, 128])
-def test_values_behind_masked_keys_do_not_leak(hip, h):
+def test_values_behind_masked_keys_do_not_leak(hip, dtype, h):
     # key 40 is not finite: queries before it and (masked) all queries of batch row 1 never see it
     b, t = 2, 300
-    q, k, v = _inputs(b, h, h, t, t, 128, torch.bfloat16, seed=3)
+    q, k, v = _inputs(b, h, h, t, t, 128, dtype, seed=3)
     valid = torch.ones(b, t, dtype=torch.bool)
     valid[1, 40] = False
     ref = torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid)
@@ -65,11 +70,11 @@ def test_values_behind_masked_keys_do_not_leak(hip, h):
         v2 = v.clone()
         v2[:, :, 40, 7] = bad
         out = _run(q, k, v2, valid)
-        _compare(out[0, :, :40], ref[0, :, :40], torch.bfloat16)
-        _compare(out[1], ref[1], torch.bfloat16)
+        _compare(out[0, :, :40], ref[0, :, :40], dtype)
+        _compare(out[1], ref[1], dtype)
         seen = out[0, :, 40:, 7].float()
         assert (torch.isnan(seen) if bad != bad else seen == bad).all()
-        _compare(out[0, :, 40:, 8:], ref[0, :, 40:, 8:], torch.bfloat16)
+        _compare(out[0, :, 40:, 8:], ref[0, :, 40:, 8:], dtype)
 
 
 def test_unaligned_rows_and_large_scores(hip):
