@@ -304,6 +304,20 @@ int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st
                          int32_t dtype, void* out, int64_t o_sb, int64_t o_sh, int64_t o_st, void* stream);
 
 /*
+ * RMSNorm of `rows` contiguous rows of `dim` elements (reference src/minillm/model/llama.py:37-49):
+ * out = weight * T(x * rsqrt(mean(x^2) + eps)), fp32 arithmetic, T the 16-bit `dtype` (BF16 or F16).  With
+ * `residual` and `sum` (both or neither), x is first replaced by T(x + residual), which is written to `sum`
+ * (reference llama.py:125, the sum before the second norm).  dim a multiple of 8, pointers 16-byte aligned; `out`
+ * and `sum` overlap no input.
+ */
+int mllm_rms_norm(const void* x, const void* residual, const void* weight, int64_t rows, int64_t dim, float eps,
+                  int32_t dtype, void* sum, void* out, void* stream);
+
+/* out = T(silu(gate) * up) over n contiguous elements, fp32 arithmetic (reference llama.py:117-120); n a multiple of
+ * 8, pointers 16-byte aligned. */
+int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_t dtype, void* out, void* stream);
+
+/*
  * fp8 KV pool.  No counterpart in the reference's code: it is the reference's planned fp8 KV cache
  * (docs/distributed_inference_plan.md:310, milestone M9b), which halves the bytes decode streams.
  * The pool has the layout above with one byte per element, OCP float8 e4m3fn (torch.float8_e4m3fn),

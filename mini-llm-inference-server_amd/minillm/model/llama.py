@@ -4,8 +4,9 @@ checkpoints load by name).
 
 The hot path's call site is `LlamaAttention.forward` on a ragged paged step: q/k/v of the N new tokens
 go to `backend.forward(q[N,H,Dh], k[N,Hkv,Dh], v[N,Hkv,Dh], k_pool[layer], v_pool[layer], meta)`,
-which appends k/v to the pool and returns the attention output.  GEMMs, RMSNorm, RoPE and SwiGLU stay
-in PyTorch.  Without a cache (kv_cache None) the contiguous `backend.prefill` path runs instead.
+which appends k/v to the pool and returns the attention output.  The matrix products and RoPE's table stay in
+PyTorch; RMSNorm, the residual sum before it and SwiGLU run as one kernel each where `kernels.usable` allows
+it (16-bit tensors, no gradients), else as torch expressions.  Without a cache (kv_cache None) the contiguous `backend.prefill` path runs instead.
 """
 
 from __future__ import annotations
@@ -15,6 +16,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from ..attention import AttentionBackend, get_backend
+from . import kernels
 from .config import LlamaConfig
 from .rope import compute_inv_freq
 
@@ -27,6 +29,8 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x * rsqrt(mean(x^2) + eps) computed in float32, cast back, then scaled by the weight."""
+        if kernels.usable(x) and kernels.norm_ok(x, self.weight):
+            return kernels.rms_norm(x, self.weight, self.eps)
         h = x.float()
         h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + self.eps)
         return self.weight * h.to(x.dtype)
@@ -111,7 +115,8 @@ class LlamaMLP(nn.Module):
         self.down_proj = nn.Linear(f, d, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+        gate, up = self.gate_proj(x), self.up_proj(x)
+        return self.down_proj(kernels.silu_mul(gate, up) if kernels.silu_mul_ok(gate, up) else F.silu(gate) * up)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -123,8 +128,15 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(config)
 
     def forward(self, x, cos, sin, kv_cache=None, key_valid=None):
-        x = x + self.self_attn(self.input_layernorm(x), cos, sin, kv_cache, key_valid)
-        return x + self.mlp(self.post_attention_layernorm(x))
+        attn = self.self_attn(self.input_layernorm(x), cos, sin, kv_cache, key_valid)
+        norm = self.post_attention_layernorm
+        if kernels.usable(x) and kernels.bare(norm, RMSNorm) and kernels.norm_ok(x, norm.weight) \
+                and kernels.sum_ok(x, attn):
+            x, h = kernels.add_rms_norm(x, attn, norm.weight, norm.eps)
+        else:
+            x = x + attn
+            h = norm(x)
+        return x + self.mlp(h)
 
 
 class LlamaModel(nn.Module):

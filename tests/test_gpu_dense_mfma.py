@@ -29,7 +29,7 @@ def _compare(out, ref, dtype):
     if dtype == torch.float32:  # sums of up to 1,000 terms: a few times 2^-24 of the terms' size
         torch.testing.assert_close(out.double(), ref, rtol=1e-5, atol=1e-5)
         return
-    # the output's own rounding (2^-9 bf16, 2^-12 fp16 of the value, doubled), plus the weights' 16 bits or more:
+    # the output's own rounding (2^-8 bf16, 2^-11 fp16 of the value), plus the weights' 16 bits or more:
     # 2^-16 of |v| <= 6, and fp32 sums: 2e-4 covers both
     torch.testing.assert_close(out.double(), ref, rtol=2 ** (-8 if dtype == torch.bfloat16 else -11), atol=2e-4)
 
