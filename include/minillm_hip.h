@@ -318,6 +318,26 @@ int mllm_rms_norm(const void* x, const void* residual, const void* weight, int64
 int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_t dtype, void* out, void* stream);
 
 /*
+ * Linear layers of few rows (reference src/minillm/model/llama.py:75-120): x [m, k] contiguous, weights [n, k] contiguous
+ * as torch.nn.Linear holds them, m <= 64, k a multiple of 256, n multiples of 16, BF16 or F16, fp32 sums, 16-byte
+ * aligned pointers.  A row's result depends neither on the other rows nor on m.
+ *
+ * mllm_linear_partial: up to three weights that share x (w1, w2 with n1 = n2 = 0 when absent), K cut into `ksplit`
+ * parts: part[ksplit][m][n0 + n1 + n2] fp32, whose sum over the parts is x . w^T.
+ * mllm_sum_partials: out [rows, dim] = T(residual + sum of the parts) (residual may be NULL).
+ * mllm_sum_partials_norm: sum = T(residual + sum of the parts) and out = its RMSNorm (mllm_rms_norm).
+ * mllm_linear_swiglu: out [m, n] = T(silu(x . gate^T) * (x . up^T)).
+ */
+int mllm_linear_partial(const void* x, int64_t m, int64_t k, const void* w0, int64_t n0, const void* w1, int64_t n1,
+                        const void* w2, int64_t n2, int32_t ksplit, float* part, int32_t dtype, void* stream);
+int mllm_sum_partials(const float* part, int32_t ksplit, int64_t rows, int64_t dim, const void* residual,
+                      int32_t dtype, void* out, void* stream);
+int mllm_sum_partials_norm(const float* part, int32_t ksplit, const void* residual, const void* weight, int64_t rows,
+                           int64_t dim, float eps, int32_t dtype, void* sum, void* out, void* stream);
+int mllm_linear_swiglu(const void* x, int64_t m, int64_t k, const void* gate, const void* up, int64_t n,
+                       int32_t dtype, void* out, void* stream);
+
+/*
  * fp8 KV pool.  No counterpart in the reference's code: it is the reference's planned fp8 KV cache
  * (docs/distributed_inference_plan.md:310, milestone M9b), which halves the bytes decode streams.
  * The pool has the layout above with one byte per element, OCP float8 e4m3fn (torch.float8_e4m3fn),

@@ -36,15 +36,32 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
 // One workgroup per row: out = w * T(x * rsqrt(mean(x^2) + eps)), the cast before the weight as the module states
 // it.  With ADD, x is first replaced by T(x + y), which is also written to `sum`.  A row of up to kKeep x 2,048
 // elements stays in registers between the two passes, a longer one is read again (with ADD, from `sum`: each thread
-// reads what it wrote).
+// reads what it wrote).  With SPLIT, y is the fp32 sum of the row's `ksplit` partial sums (mllm_linear_partial).
 constexpr int kNormThreads = 256;
 constexpr int kKeep = 4;  // 16-byte pieces per thread kept in registers
 
-template <typename T, bool ADD>
+// Adds piece i (8 columns) of the parts to f, in their order.
+__device__ __forceinline__ void add_parts(const float* part, int ksplit, int64_t stride, int64_t at, float (&f)[8]) {
+  f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll 8
+  for (int k = 0; k < ksplit; ++k) {
+    lo += *reinterpret_cast<const f32x4*>(part + k * stride + at);
+    hi += *reinterpret_cast<const f32x4*>(part + k * stride + at + 4);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    f[e] += lo[e];
+    f[4 + e] += hi[e];
+  }
+}
+
+template <typename T, bool ADD, bool SPLIT = false>
 __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(const uint16_t* __restrict__ x,
                                                                 const uint16_t* __restrict__ y,
                                                                 const uint16_t* __restrict__ w, uint16_t* sum,
-                                                                uint16_t* __restrict__ out, int64_t dim, float eps) {
+                                                                uint16_t* __restrict__ out, int64_t dim, float eps,
+                                                                const float* __restrict__ part = nullptr,
+                                                                int ksplit = 0, int64_t part_stride = 0) {
   __shared__ float red[kNormThreads / 64];
   const int64_t row = (int64_t)blockIdx.x * dim;
   const int pieces = (int)(dim / 8);
@@ -55,10 +72,14 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(const uint16_t* 
     float f[8];
     unpack8<T>(v, f);
     if constexpr (ADD) {
-      float g[8];
-      unpack8<T>(ld16(y + row + 8 * (int64_t)i), g);
+      if constexpr (SPLIT) {
+        add_parts(part, ksplit, part_stride, row + 8 * (int64_t)i, f);
+      } else {
+        float g[8];
+        unpack8<T>(ld16(y + row + 8 * (int64_t)i), g);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] += g[e];
+        for (int e = 0; e < 8; ++e) f[e] += g[e];
+      }
       v = pack8<T>(f);
       st16(sum + row + 8 * (int64_t)i, v);
       unpack8<T>(v, f);
@@ -112,6 +133,19 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
   st16(out + 8 * i, pack8<T>(g));
 }
 
+// out = T(residual + the sum of the parts) over n elements (a multiple of 8); no residual: the sum alone.
+template <typename T>
+__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ part, int ksplit, int64_t n,
+                                                           const uint16_t* __restrict__ residual,
+                                                           uint16_t* __restrict__ out) {
+  const int64_t i = 8 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (i >= n) return;
+  float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (residual) unpack8<T>(ld16(residual + i), f);
+  add_parts(part, ksplit, n, i, f);
+  st16(out + i, pack8<T>(f));
+}
+
 }  // namespace
 }  // namespace mllm
 
@@ -159,4 +193,50 @@ extern "C" int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_
   else
     silu_mul_kernel<F16><<<grid, 256, 0, st>>>((const uint16_t*)gate, (const uint16_t*)up, (uint16_t*)out, n / 8);
   return check_launch("mllm_silu_mul");
+}
+
+extern "C" int mllm_sum_partials(const float* part, int32_t ksplit, int64_t rows, int64_t dim, const void* residual,
+                                 int32_t dtype, void* out, void* stream) {
+  using namespace mllm;
+  MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
+               "mllm_sum_partials: dtype must be bfloat16 or float16");
+  MLLM_REQUIRE(ksplit >= 1 && rows >= 0 && dim > 0 && dim % 8 == 0 && rows < (1ll << 31) && dim < (1ll << 31),
+               MLLM_ERR_INVALID, "mllm_sum_partials: bad sizes");
+  if (rows == 0) return MLLM_OK;
+  MLLM_REQUIRE(part && out, MLLM_ERR_INVALID, "mllm_sum_partials: null pointer");
+  MLLM_REQUIRE(((uintptr_t)part | (uintptr_t)residual | (uintptr_t)out) % 16 == 0, MLLM_ERR_UNSUPPORTED,
+               "mllm_sum_partials: operands must be 16-byte aligned");
+  const int64_t n = rows * dim, groups = (n / 8 + 255) / 256;
+  MLLM_REQUIRE(groups < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_sum_partials: too many elements");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (dtype == MLLM_DTYPE_BF16)
+    sum_partials_kernel<BF16><<<(unsigned)groups, 256, 0, st>>>(part, ksplit, n, (const uint16_t*)residual, (uint16_t*)out);
+  else
+    sum_partials_kernel<F16><<<(unsigned)groups, 256, 0, st>>>(part, ksplit, n, (const uint16_t*)residual, (uint16_t*)out);
+  return check_launch("mllm_sum_partials");
+}
+
+extern "C" int mllm_sum_partials_norm(const float* part, int32_t ksplit, const void* residual, const void* weight,
+                                      int64_t rows, int64_t dim, float eps, int32_t dtype, void* sum, void* out,
+                                      void* stream) {
+  using namespace mllm;
+  MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
+               "mllm_sum_partials_norm: dtype must be bfloat16 or float16");
+  MLLM_REQUIRE(ksplit >= 1 && rows >= 0 && dim > 0 && dim % 8 == 0 && rows < (1ll << 31) && dim < (1ll << 31),
+               MLLM_ERR_INVALID, "mllm_sum_partials_norm: bad sizes");
+  if (rows == 0) return MLLM_OK;
+  MLLM_REQUIRE(part && residual && weight && sum && out, MLLM_ERR_INVALID, "mllm_sum_partials_norm: null pointer");
+  MLLM_REQUIRE(((uintptr_t)part | (uintptr_t)residual | (uintptr_t)weight | (uintptr_t)sum | (uintptr_t)out) % 16 == 0,
+               MLLM_ERR_UNSUPPORTED, "mllm_sum_partials_norm: rows must be 16-byte aligned");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  auto launch = [&](auto tag) {
+    rms_norm_kernel<decltype(tag), true, true><<<(unsigned)rows, kNormThreads, 0, st>>>(
+        (const uint16_t*)residual, nullptr, (const uint16_t*)weight, (uint16_t*)sum, (uint16_t*)out, dim, eps, part,
+        ksplit, rows * dim);
+  };
+  if (dtype == MLLM_DTYPE_BF16)
+    launch(BF16{});
+  else
+    launch(F16{});
+  return check_launch("mllm_sum_partials_norm");
 }

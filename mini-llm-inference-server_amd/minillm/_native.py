@@ -66,6 +66,10 @@ SIGNATURES = {
                                             _p]),
     "mllm_rms_norm": (ctypes.c_int, [_p, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
     "mllm_silu_mul": (ctypes.c_int, [_p, _p, _i64, _i32, _p, _p]),
+    "mllm_linear_partial": (ctypes.c_int, [_p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i32, _p, _i32, _p]),
+    "mllm_sum_partials": (ctypes.c_int, [_p, _i32, _i64, _i64, _p, _i32, _p, _p]),
+    "mllm_sum_partials_norm": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
+    "mllm_linear_swiglu": (ctypes.c_int, [_p, _i64, _i64, _p, _p, _i64, _i32, _p, _p]),
     # fp8 (e4m3fn) pools with per-tensor k_scale / v_scale
     "mllm_kv_append_fp8": (ctypes.c_int, [_p, _i64, _i64, _p, _i64, _i64, _i32, _p, _p, _i64, _i32, _i32, _p, _i64, _f32,
                                           _f32, _p]),

@@ -1,4 +1,5 @@
-"""The decoder layer's kernels around its matrix products (csrc/norm.hip), for the model's inference path.
+"""The decoder layer's kernels around its matrix products (csrc/norm.hip) and its products on few rows
+(csrc/linear.hip), for the model's inference path.
 
 `usable(x)` says whether a call may take them: a plain 16-bit CUDA tensor on the current device, gradients off, and
 nothing active that follows torch's operations (tracing, compilation, autocast, function or dispatch modes, functorch
@@ -81,4 +82,85 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     out = torch.empty_like(gate)
     _native.lib().call("mllm_silu_mul", gate.data_ptr(), up.data_ptr(), gate.numel(), _native.dtype_code(gate.dtype),
                        out.data_ptr(), _native.stream_ptr(gate.device))
+    return out
+
+
+# ---------------------------------------------------------------- linear layers of few rows
+
+SMALL_ROWS = 64  # rows of x the kernels take
+TILE = 128  # weight rows per workgroup
+CHUNK = 256  # K granularity
+FULL_CHIP = 256  # workgroups that give every CU of the full chip one
+
+
+def small_rows(x: torch.Tensor) -> bool:
+    """Whether x [..., K] has few enough rows for these kernels.  The line lies at 64, what their accumulators and LDS are
+    laid out for; up to it each measured faster than the library product (csrc/linear.hip), with q, k, v and gate,
+    up sharing launches on top."""
+    return type(x) is torch.Tensor and 0 < x.numel() <= SMALL_ROWS * x.shape[-1] and _rows_ok(x, x)
+
+
+def weights_ok(like: torch.Tensor, k: int, *linears) -> bool:
+    """Whether the few-row kernels take these layers for operands of `k` columns with the type and device of `like`."""
+    if k % CHUNK:
+        return False
+    for m in linears:
+        if not bare(m, torch.nn.Linear) or m.bias is not None:
+            return False
+        w = m.weight
+        if w.shape[1] != k or w.shape[0] % 16 or not _plain_weight(w, like):
+            return False
+    return True
+
+
+def ksplit(k: int, *rows: int) -> int:
+    """Parts of K per output tile: as many as give every CU about one workgroup (the launch is then one round: the o
+    projection of Llama-3.1-8B 9.4 us at 8 parts against 12.5 at 4, q, k and v 13.7 at 5 against 14.3 at 4), at most 8
+    (each part's sums are written and read again) and none shorter than two chunks."""
+    tiles = sum(-(-n // TILE) for n in rows)
+    return max(1, min(FULL_CHIP // tiles, 8, k // CHUNK // 2))
+
+
+def _partial(x: torch.Tensor, weights) -> tuple[torch.Tensor, int, int]:
+    k = x.shape[-1]
+    m = x.numel() // k
+    rows = [w.shape[0] for w in weights]
+    ks = ksplit(k, *rows)
+    part = torch.empty(ks * m * sum(rows), dtype=torch.float32, device=x.device)
+    args = []
+    for w in weights:
+        args += (w.data_ptr(), w.shape[0])
+    args += (None, 0) * (3 - len(weights))
+    _native.lib().call("mllm_linear_partial", x.data_ptr(), m, k, *args, ks, part.data_ptr(),
+                       _native.dtype_code(x.dtype), _native.stream_ptr(x.device))
+    return part, ks, m
+
+
+def linear(x: torch.Tensor, *weights, residual: torch.Tensor | None = None) -> torch.Tensor:
+    """x . w^T of each weight side by side, [..., sum of rows] (plus `residual`, of that shape)."""
+    part, ks, m = _partial(x, weights)
+    n = part.numel() // (ks * m)
+    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    _native.lib().call("mllm_sum_partials", part.data_ptr(), ks, m, n,
+                       None if residual is None else residual.data_ptr(), _native.dtype_code(x.dtype), out.data_ptr(),
+                       _native.stream_ptr(x.device))
+    return out
+
+
+def linear_add_norm(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor, norm: torch.Tensor, eps: float):
+    """(residual + x . w^T, its RMSNorm)."""
+    part, ks, m = _partial(x, (weight,))
+    total, out = torch.empty_like(residual), torch.empty_like(residual)
+    _native.lib().call("mllm_sum_partials_norm", part.data_ptr(), ks, residual.data_ptr(), norm.data_ptr(), m,
+                       weight.shape[0], eps, _native.dtype_code(x.dtype), total.data_ptr(), out.data_ptr(),
+                       _native.stream_ptr(x.device))
+    return total, out
+
+
+def linear_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    """silu(x . gate^T) * (x . up^T)."""
+    k, n = x.shape[-1], gate.shape[0]
+    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    _native.lib().call("mllm_linear_swiglu", x.data_ptr(), x.numel() // k, k, gate.data_ptr(), up.data_ptr(), n,
+                       _native.dtype_code(x.dtype), out.data_ptr(), _native.stream_ptr(x.device))
     return out

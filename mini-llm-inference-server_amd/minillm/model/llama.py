@@ -4,9 +4,9 @@ checkpoints load by name).
 
 The hot path's call site is `LlamaAttention.forward` on a ragged paged step: q/k/v of the N new tokens
 go to `backend.forward(q[N,H,Dh], k[N,Hkv,Dh], v[N,Hkv,Dh], k_pool[layer], v_pool[layer], meta)`,
-which appends k/v to the pool and returns the attention output.  The matrix products and RoPE's table stay in
-PyTorch; RMSNorm, the residual sum before it and SwiGLU run as one kernel each where `kernels.usable` allows
-it (16-bit tensors, no gradients), else as torch expressions.  Without a cache (kv_cache None) the contiguous `backend.prefill` path runs instead.
+which appends k/v to the pool and returns the attention output.  Where `kernels.usable` allows it (16-bit
+tensors, no gradients) RMSNorm, the residual sum before it and SwiGLU run as one kernel each, and the
+products of steps of up to 64 rows as few-row kernels; everything else stays in PyTorch.  Without a cache (kv_cache None) the contiguous `backend.prefill` path runs instead.
 """
 
 from __future__ import annotations
@@ -80,11 +80,20 @@ class LlamaAttention(nn.Module):
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kv_cache=None,
                 key_valid: torch.Tensor | None = None) -> torch.Tensor:
+        return self.o_proj(self.attend(x, cos, sin, kv_cache, key_valid))
+
+    def attend(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kv_cache=None,
+               key_valid: torch.Tensor | None = None) -> torch.Tensor:
+        """The attention output before o_proj, [B, T, H Dh]."""
         b, t, _ = x.shape
         dh = self.config.head_dim
-        q = self.q_proj(x).view(b, t, -1, dh).transpose(1, 2)
-        k = self.k_proj(x).view(b, t, -1, dh).transpose(1, 2)
-        v = self.v_proj(x).view(b, t, -1, dh).transpose(1, 2)
+        q_proj, k_proj, v_proj = self.q_proj, self.k_proj, self.v_proj
+        if kernels.usable(x) and kernels.small_rows(x) and kernels.weights_ok(x, x.shape[-1], q_proj, k_proj, v_proj):
+            qkv = kernels.linear(x, q_proj.weight, k_proj.weight, v_proj.weight)
+            q, k, v = qkv.split((q_proj.weight.shape[0], k_proj.weight.shape[0], v_proj.weight.shape[0]), dim=-1)
+        else:
+            q, k, v = q_proj(x), k_proj(x), v_proj(x)
+        q, k, v = (p.view(b, t, -1, dh).transpose(1, 2) for p in (q, k, v))
         if getattr(kv_cache, "ragged", False):
             # ragged step: one row of every sequence's new tokens -> [N, heads, Dh] views for the backend
             layer = self.layer_idx
@@ -98,12 +107,12 @@ class LlamaAttention(nn.Module):
                 q, k = apply_rotary(q, cos, sin), apply_rotary(k, cos, sin)
                 out = self.backend.forward(q[0].transpose(0, 1), k[0].transpose(0, 1), v[0].transpose(0, 1), *pools,
                                            **scales)
-            return self.o_proj(out.reshape(b, t, -1))
+            return out.reshape(b, t, -1)
         q, k = apply_rotary(q, cos, sin), apply_rotary(k, cos, sin)
         if kv_cache is not None:
             raise ValueError("only paged ragged caches (PagedStep) are supported")
         out = self.backend.prefill(q, k, v, key_valid=key_valid)
-        return self.o_proj(out.transpose(1, 2).reshape(b, t, -1))
+        return out.transpose(1, 2).reshape(b, t, -1)
 
 
 class LlamaMLP(nn.Module):
@@ -128,15 +137,36 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(config)
 
     def forward(self, x, cos, sin, kv_cache=None, key_valid=None):
-        attn = self.self_attn(self.input_layernorm(x), cos, sin, kv_cache, key_valid)
         norm = self.post_attention_layernorm
-        if kernels.usable(x) and kernels.bare(norm, RMSNorm) and kernels.norm_ok(x, norm.weight) \
-                and kernels.sum_ok(x, attn):
-            x, h = kernels.add_rms_norm(x, attn, norm.weight, norm.eps)
+        fused = kernels.usable(x) and kernels.bare(norm, RMSNorm) and kernels.norm_ok(x, norm.weight)
+        if fused and kernels.small_rows(x) and self._small_ok(x):
+            attn, mlp = self.self_attn, self.mlp
+            out = attn.attend(self.input_layernorm(x), cos, sin, kv_cache, key_valid)
+            if kernels.small_rows(out) and kernels.weights_ok(out, out.shape[-1], attn.o_proj):
+                x, h = kernels.linear_add_norm(out, attn.o_proj.weight, x, norm.weight, norm.eps)
+                h = kernels.linear_swiglu(h, mlp.gate_proj.weight, mlp.up_proj.weight)
+                return kernels.linear(h, mlp.down_proj.weight, residual=x)
+            out = attn.o_proj(out)
         else:
-            x = x + attn
+            out = self.self_attn(self.input_layernorm(x), cos, sin, kv_cache, key_valid)
+        if fused and kernels.sum_ok(x, out):
+            x, h = kernels.add_rms_norm(x, out, norm.weight, norm.eps)
+        else:
+            x = x + out
             h = norm(x)
         return x + self.mlp(h)
+
+    def _small_ok(self, x: torch.Tensor) -> bool:
+        """Whether everything behind the attention may run as the few-row kernels: submodules without hooks, plain
+        weights that fit together."""
+        attn, mlp = self.self_attn, self.mlp
+        if not (kernels.bare(attn, LlamaAttention) and kernels.bare(mlp, LlamaMLP)):
+            return False
+        d, gate, up, down = x.shape[-1], mlp.gate_proj, mlp.up_proj, mlp.down_proj
+        if not (kernels.weights_ok(x, d, gate, up) and gate.weight.shape == up.weight.shape):
+            return False
+        return kernels.weights_ok(x, gate.weight.shape[0], down) and down.weight.shape[0] == d \
+            and attn.o_proj.weight.shape[0] == d
 
 
 class LlamaModel(nn.Module):

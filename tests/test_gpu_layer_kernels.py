@@ -68,3 +68,86 @@ def test_torch_path_kept(hip):
     assert kernels.bare(norm, RMSNorm)
     norm.register_forward_hook(lambda *a: None)
     assert not kernels.bare(norm, RMSNorm)
+
+
+def _ref(x, w):
+    return x.double() @ w.double().t()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,k,rows", [(1, 256, (16,)), (15, 512, (144, 16)), (16, 4096, (4096, 1024, 1024)),
+                                      (17, 1024, (272,)), (33, 2048, (128, 112, 240)), (48, 768, (4096,)),
+                                      (49, 14336, (256,)), (64, 4096, (1008,))])
+def test_linear_of_few_rows(hip, dtype, m, k, rows):
+    from minillm.model import kernels
+
+    x, res = _randn((1, m, k), dtype, 8), _randn((1, m, sum(rows)), dtype, 9)
+    ws = [_randn((n, k), dtype, 10 + i, 0.05) for i, n in enumerate(rows)]
+    out, plus = kernels.linear(x, *ws), kernels.linear(x, *ws, residual=res)
+    ref = torch.cat([_ref(x, w) for w in ws], dim=-1)
+    # one rounding, and the fp32 sums' error: k terms of some 0.05, each addition off by at most 2^-24 of a partial sum
+    # of at most some 10, in random directions: sqrt(14,336) x 6e-7 < 1e-4
+    torch.testing.assert_close(out.double(), ref, rtol=1.01 * EPS[dtype], atol=1e-4)
+    torch.testing.assert_close(plus.double(), ref + res.double(), rtol=1.01 * EPS[dtype], atol=1e-4)
+    # a row's result is the same alone, and whatever rows are beside it
+    assert torch.equal(kernels.linear(x[:, -1:].contiguous(), *ws), out[:, -1:])
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 256, 16), (16, 512, 80), (37, 4096, 14336), (64, 1024, 144)])
+def test_linear_swiglu_and_norm_behind_a_product(hip, m, k, n):
+    from minillm.model import kernels
+
+    dtype = torch.bfloat16
+    x = _randn((1, m, k), dtype, 11)
+    gate, up = _randn((n, k), dtype, 12, 0.05), _randn((n, k), dtype, 13, 0.05)
+    g = _ref(x, gate)
+    # the sums' fp32 error (1e-5 and less) moves silu by less than 1.1 times itself, times |up| of some units
+    torch.testing.assert_close(kernels.linear_swiglu(x, gate, up).double(), g / (1 + torch.exp(-g)) * _ref(x, up),
+                               rtol=1.01 * EPS[dtype], atol=1e-3)
+    res, w = _randn((1, m, n), dtype, 14), _randn((n,), dtype, 15) * 0.1 + 1
+    total, out = kernels.linear_add_norm(x, gate, res, w, 1e-5)
+    torch.testing.assert_close(total.double(), res.double() + g, rtol=1.01 * EPS[dtype], atol=1e-4)
+    d = total.double()
+    torch.testing.assert_close(out.double(), w.double() * (d * torch.rsqrt(d.square().mean(-1, keepdim=True) + 1e-5)),
+                               rtol=2.02 * EPS[dtype], atol=1e-6)
+
+
+def test_few_row_layers_keep_hooks_biases_and_wide_rows(hip):
+    from minillm.model import kernels
+
+    lin = torch.nn.Linear(256, 32, bias=False, device=DEV, dtype=torch.bfloat16)
+    x = _randn((1, 64, 256), torch.bfloat16, 16)
+    with torch.no_grad():
+        assert kernels.small_rows(x) and kernels.weights_ok(x, 256, lin)
+        assert not kernels.small_rows(_randn((1, 65, 256), torch.bfloat16, 17)) and not kernels.weights_ok(x, 128, lin)
+        assert not kernels.weights_ok(x.half(), 256, lin)
+        assert not kernels.weights_ok(x, 256, torch.nn.Linear(256, 32, device=DEV, dtype=torch.bfloat16))
+        assert not kernels.weights_ok(x, 256, torch.nn.Linear(256, 24, bias=False, device=DEV, dtype=torch.bfloat16))
+    handle = lin.register_forward_pre_hook(lambda *a: None)
+    assert not kernels.weights_ok(x, 256, lin)
+    handle.remove()
+    assert kernels.weights_ok(x, 256, lin)
+
+
+@pytest.mark.parametrize("part", ["o_proj", "mlp", "post_attention_layernorm"])
+def test_decoder_layer_with_a_hook_calls_it(hip, part):
+    from minillm.attention import get_backend
+    from minillm.model.config import LlamaConfig
+    from minillm.model.llama import LlamaDecoderLayer, LlamaModel, random_init_  # noqa: F401
+
+    cfg = LlamaConfig(vocab_size=64, hidden_size=512, intermediate_size=768, num_hidden_layers=1, num_attention_heads=4,
+                      num_key_value_heads=2, head_dim=128, rms_norm_eps=1e-5, rope_theta=1e4, rope_scaling=None,
+                      max_position_embeddings=512)
+    layer = LlamaDecoderLayer(cfg, get_backend("hip"), 0).to(DEV, torch.bfloat16)
+    x = _randn((2, 9, 512), torch.bfloat16, 18)
+    ang = torch.randn(2, 9, 128, device=DEV)
+    with torch.inference_mode():
+        cos, sin = ang.cos().bfloat16(), ang.sin().bfloat16()
+        plain = layer(x, cos, sin)
+        seen = []
+        target = layer.self_attn.o_proj if part == "o_proj" else getattr(layer, part)
+        target.register_forward_hook(lambda *a: seen.append(1))
+        hooked = layer(x, cos, sin)
+    assert seen == [1]
+    # the two paths round at different places: a few bf16 roundings of values of some units
+    torch.testing.assert_close(plain.float(), hooked.float(), rtol=4 * EPS[torch.bfloat16], atol=0.03)
