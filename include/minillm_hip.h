@@ -322,12 +322,14 @@ int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_t dtype, vo
  * as torch.nn.Linear holds them, m <= 64, k a multiple of 256, n multiples of 16, BF16 or F16, fp32 sums, 16-byte
  * aligned pointers.  A row's result depends neither on the other rows nor on m.
  *
+ * mllm_linear_ksplit: the number of parts of K that fills the chip for these weights (>= 1).
  * mllm_linear_partial: up to three weights that share x (w1, w2 with n1 = n2 = 0 when absent), K cut into `ksplit`
  * parts: part[ksplit][m][n0 + n1 + n2] fp32, whose sum over the parts is x . w^T.
  * mllm_sum_partials: out [rows, dim] = T(residual + sum of the parts) (residual may be NULL).
  * mllm_sum_partials_norm: sum = T(residual + sum of the parts) and out = its RMSNorm (mllm_rms_norm).
  * mllm_linear_swiglu: out [m, n] = T(silu(x . gate^T) * (x . up^T)).
  */
+int mllm_linear_ksplit(int64_t k, int64_t n0, int64_t n1, int64_t n2);
 int mllm_linear_partial(const void* x, int64_t m, int64_t k, const void* w0, int64_t n0, const void* w1, int64_t n1,
                         const void* w2, int64_t n2, int32_t ksplit, float* part, int32_t dtype, void* stream);
 int mllm_sum_partials(const float* part, int32_t ksplit, int64_t rows, int64_t dim, const void* residual,
@@ -336,6 +338,22 @@ int mllm_sum_partials_norm(const float* part, int32_t ksplit, const void* residu
                            int64_t dim, float eps, int32_t dtype, void* sum, void* out, void* stream);
 int mllm_linear_swiglu(const void* x, int64_t m, int64_t k, const void* gate, const void* up, int64_t n,
                        int32_t dtype, void* out, void* stream);
+
+/*
+ * A whole decoder layer of a paged step of at most 64 rows in one host call (reference src/minillm/model/llama.py:117-127):
+ *   h = RMSNorm(x); q, k, v = h . w^T; the step's RoPE, append and attention (mllm_attention_forward);
+ *   x2 = x + attn . wo^T; out = x2 + SwiGLU(RMSNorm(x2)) . down^T
+ * as the launches of the entry points above, in that order on `stream`, with their limits; x and out [N, hidden], weights as
+ * torch.nn.Linear holds them.  `scratch`: mllm_decoder_layer_scratch_bytes bytes, 256-byte aligned, not shared with
+ * a call that may run at the same time.
+ */
+int64_t mllm_decoder_layer_scratch_bytes(int64_t rows, int64_t hidden, int64_t ffn, int32_t num_heads,
+                                         int32_t num_kv_heads, int32_t head_dim);
+int mllm_decoder_layer(const mllm_layer_step* step, const void* x, int64_t hidden, const void* norm1, float eps1,
+                       const void* wq, const void* wk, const void* wv, const void* wo, const void* norm2, float eps2,
+                       const void* gate, const void* up, const void* down, int64_t ffn, const void* cos,
+                       const void* sin, int64_t cs_stride_tok, void* k_cache, void* v_cache, float k_scale,
+                       float v_scale, void* scratch, int64_t scratch_bytes, void* out, void* stream);
 
 /*
  * fp8 KV pool.  No counterpart in the reference's code: it is the reference's planned fp8 KV cache

@@ -16,6 +16,8 @@
 //   o       9.4 / 10.5 / 12.2 (15.8 / 13.2 / 15.2)    down      23.7 / 24.7 / 27.4 (25.0 / 29.5 / 38.8)
 // gate and up stream 5.4 TB/s.  Tiles of 64 rows with two wavefronts along K measured 13.1, 9.2, 49.0 and 23.6 us at
 // 8 rows.  A row's result depends neither on the other rows nor on M.
+#include <initializer_list>
+
 #include "common.h"
 
 namespace mllm {
@@ -168,6 +170,19 @@ int check_operands(const char* fn, const void* x, int64_t m, int64_t k, int32_t 
 
 }  // namespace
 }  // namespace mllm
+
+// Parts of K per output tile: as many as give every CU of the full chip (256) about one workgroup, so that the launch
+// is one round (o of Llama-3.1-8B 9.4 us at 8 parts against 12.5 at 4; q, k and v 13.7 at 5 against 14.3 at 4), at
+// most 8 (each part's sums are written and read again) and none shorter than two chunks.
+extern "C" int mllm_linear_ksplit(int64_t k, int64_t n0, int64_t n1, int64_t n2) {
+  using namespace mllm;
+  int64_t tiles = 0;
+  for (const int64_t n : {n0, n1, n2}) tiles += (n + kTileRows - 1) / kTileRows;
+  int64_t ks = tiles > 0 ? 256 / tiles : 1;
+  if (ks > 8) ks = 8;
+  if (ks > k / kChunk / 2) ks = k / kChunk / 2;
+  return ks < 1 ? 1 : (int)ks;
+}
 
 extern "C" int mllm_linear_partial(const void* x, int64_t m, int64_t k, const void* w0, int64_t n0, const void* w1,
                                    int64_t n1, const void* w2, int64_t n2, int32_t ksplit, float* part, int32_t dtype,

@@ -70,6 +70,10 @@ SIGNATURES = {
     "mllm_sum_partials": (ctypes.c_int, [_p, _i32, _i64, _i64, _p, _i32, _p, _p]),
     "mllm_sum_partials_norm": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
     "mllm_linear_swiglu": (ctypes.c_int, [_p, _i64, _i64, _p, _p, _i64, _i32, _p, _p]),
+    "mllm_linear_ksplit": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
+    "mllm_decoder_layer_scratch_bytes": (ctypes.c_int64, [_i64, _i64, _i64, _i32, _i32, _i32]),
+    "mllm_decoder_layer": (ctypes.c_int, [_p, _p, _i64, _p, _f32, _p, _p, _p, _p, _p, _f32, _p, _p, _p, _i64, _p, _p, _i64,
+                                          _p, _p, _f32, _f32, _p, _i64, _p, _p]),
     # fp8 (e4m3fn) pools with per-tensor k_scale / v_scale
     "mllm_kv_append_fp8": (ctypes.c_int, [_p, _i64, _i64, _p, _i64, _i64, _i32, _p, _p, _i64, _i32, _i32, _p, _i64, _f32,
                                           _f32, _p]),
@@ -127,6 +131,11 @@ class NativeLib:
 
 
 _LIB: NativeLib | None = None
+
+
+def available() -> bool:
+    """Whether the library is loaded or can be (its file is there)."""
+    return _LIB is not None or LIB_PATH.exists()
 
 
 def lib() -> NativeLib:

@@ -279,7 +279,7 @@ class HipBackend(AttentionBackend):
         are contiguous [N, H, Dh]."""
         fp8 = is_fp8(k_cache)
         plan = self.plan(meta, q.shape[1], k_cache.shape[2], q.shape[2], q.device, fp8)
-        step = self._layer_step(plan, meta, q, k_cache, fp8)
+        step = self._layer_step(plan, meta, q.shape[0], q.shape[1], q.dtype, k_cache, fp8)
         rot = cos is not None
         self._lib.check(self._attention_forward(
             step, q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
@@ -287,25 +287,32 @@ class HipBackend(AttentionBackend):
             cos.stride(0) if rot else 0, q_rot.data_ptr() if rot else None, k_cache.data_ptr(), v_cache.data_ptr(),
             k_scale, v_scale, out.data_ptr(), _native.stream_ptr(q.device)))
 
-    def _layer_step(self, plan: StepPlan, meta, q, k_cache, fp8: bool) -> int:
+    def layer_step(self, meta, n: int, num_heads: int, dtype, k_cache) -> int:
+        """Address of the step's mllm_layer_step for rows of `num_heads` query heads in `dtype` and these pools (the
+        plan is built on the first call with `meta`)."""
+        fp8 = is_fp8(k_cache)
+        plan = self.plan(meta, num_heads, k_cache.shape[2], k_cache.shape[3], k_cache.device, fp8)
+        return self._layer_step(plan, meta, n, num_heads, dtype, k_cache, fp8)
+
+    def _layer_step(self, plan: StepPlan, meta, n: int, num_heads: int, dtype, k_cache, fp8: bool) -> int:
         """Address of the plan's mllm_layer_step for these pools and this workspace."""
         ws = self._workspace
-        key = (k_cache.shape[0], k_cache.shape[1], q.dtype, fp8, ws.data_ptr() if ws is not None else 0)
+        key = (k_cache.shape[0], k_cache.shape[1], dtype, fp8, ws.data_ptr() if ws is not None else 0)
         if plan.layer_key == key:
             return plan.layer_addr
-        ws = self._workspace_for(plan.workspace_bytes, q.device)
+        ws = self._workspace_for(plan.workspace_bytes, k_cache.device)
         num_blocks, bs, hkv, dh = k_cache.shape
         step = _native.LayerStep(
-            num_blocks=num_blocks, num_tokens=q.shape[0], slot_mapping=meta.slot_mapping.data_ptr(),
+            num_blocks=num_blocks, num_tokens=n, slot_mapping=meta.slot_mapping.data_ptr(),
             qo_indptr=plan.meta_ptrs[0], kv_indptr=plan.meta_ptrs[1], kv_indices=plan.meta_ptrs[2],
             seq_lens=plan.meta_ptrs[3], decode_work=_ptr(plan.decode_work), merge_work=_ptr(plan.merge_work),
             prefill_work=_ptr(plan.prefill_work), workspace=_ptr(ws), workspace_bytes=plan.workspace_bytes,
             num_decode_work=plan.num_decode, num_merge_work=plan.num_merge, num_prefill_work=plan.num_prefill,
-            pages_per_split=plan.pages_per_split, q_tile_tokens=plan.q_tile, num_heads=q.shape[1],
-            num_kv_heads=hkv, head_dim=dh, block_size=bs, dtype=_native.dtype_code(q.dtype), kv_fp8=int(fp8),
+            pages_per_split=plan.pages_per_split, q_tile_tokens=plan.q_tile, num_heads=num_heads,
+            num_kv_heads=hkv, head_dim=dh, block_size=bs, dtype=_native.dtype_code(dtype), kv_fp8=int(fp8),
             softmax_scale=dh ** -0.5)
         plan.layer_step, plan.layer_addr = step, ctypes.addressof(step)
-        plan.layer_key = (num_blocks, bs, q.dtype, fp8, ws.data_ptr() if ws is not None else 0)
+        plan.layer_key = (num_blocks, bs, dtype, fp8, ws.data_ptr() if ws is not None else 0)
         return plan.layer_addr
 
     def _check(self, q, k, v, k_cache, v_cache, meta, k_scale=1.0, v_scale=1.0):

@@ -9,15 +9,20 @@ a submodule's `__call__` does nothing but its class's `forward`, so that a fused
 
 from __future__ import annotations
 
+import math
+
 import torch
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
 from .. import _native
+from ..attention.hip_backend import FP8, HipBackend
+from ..cache.paged import PagedKVCache, PagedStep
 
 _DTYPES = (torch.bfloat16, torch.float16)
+# what mllm_decoder_layer stands in for: a backend instance that overrides one of these is called instead
+_BACKEND_CALLS = frozenset(("forward", "forward_rotary", "run_layer", "rope_append", "append", "attend"))
 _wrapped = torch._C._functorch.is_functorch_wrapped_tensor
-_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
 
 
 def usable(x: torch.Tensor) -> bool:
@@ -25,16 +30,15 @@ def usable(x: torch.Tensor) -> bool:
             and not torch.is_autocast_enabled() and not torch._C._len_torch_dispatch_stack()
             and not torch._C._len_torch_function_stack() and not _wrapped(x) and forward_ad._current_level < 0
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and x.device.index == torch.cuda.current_device() and _native.LIB_PATH.exists())
+            and x.device.index == torch.cuda.current_device() and _native.available())
 
 
 def bare(module: torch.nn.Module, cls: type) -> bool:
-    if type(module) is not cls or "forward" in module.__dict__:
-        return False
-    if any(getattr(module, h) for h in _HOOKS):
-        return False
-    return not (_module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
-                or _module._global_backward_pre_hooks)
+    d = module.__dict__
+    return type(module) is cls and "forward" not in d \
+        and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                 or _module._global_forward_hooks or _module._global_forward_pre_hooks
+                 or _module._global_backward_hooks or _module._global_backward_pre_hooks)
 
 
 def _rows_ok(t: torch.Tensor, like: torch.Tensor) -> bool:
@@ -88,9 +92,7 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 # ---------------------------------------------------------------- linear layers of few rows
 
 SMALL_ROWS = 64  # rows of x the kernels take
-TILE = 128  # weight rows per workgroup
 CHUNK = 256  # K granularity
-FULL_CHIP = 256  # workgroups that give every CU of the full chip one
 
 
 def small_rows(x: torch.Tensor) -> bool:
@@ -105,27 +107,20 @@ def weights_ok(like: torch.Tensor, k: int, *linears) -> bool:
     if k % CHUNK:
         return False
     for m in linears:
-        if not bare(m, torch.nn.Linear) or m.bias is not None:
+        params = m.__dict__["_parameters"]
+        if not bare(m, torch.nn.Linear) or params["bias"] is not None:
             return False
-        w = m.weight
+        w = params["weight"]
         if w.shape[1] != k or w.shape[0] % 16 or not _plain_weight(w, like):
             return False
     return True
-
-
-def ksplit(k: int, *rows: int) -> int:
-    """Parts of K per output tile: as many as give every CU about one workgroup (the launch is then one round: the o
-    projection of Llama-3.1-8B 9.4 us at 8 parts against 12.5 at 4, q, k and v 13.7 at 5 against 14.3 at 4), at most 8
-    (each part's sums are written and read again) and none shorter than two chunks."""
-    tiles = sum(-(-n // TILE) for n in rows)
-    return max(1, min(FULL_CHIP // tiles, 8, k // CHUNK // 2))
 
 
 def _partial(x: torch.Tensor, weights) -> tuple[torch.Tensor, int, int]:
     k = x.shape[-1]
     m = x.numel() // k
     rows = [w.shape[0] for w in weights]
-    ks = ksplit(k, *rows)
+    ks = _native.lib().fn("mllm_linear_ksplit")(k, *rows, *(0,) * (3 - len(rows)))
     part = torch.empty(ks * m * sum(rows), dtype=torch.float32, device=x.device)
     args = []
     for w in weights:
@@ -163,4 +158,53 @@ def linear_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor) -> torc
     out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
     _native.lib().call("mllm_linear_swiglu", x.data_ptr(), x.numel() // k, k, gate.data_ptr(), up.data_ptr(), n,
                        _native.dtype_code(x.dtype), out.data_ptr(), _native.stream_ptr(x.device))
+    return out
+
+
+def decoder_layer(layer, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kv_cache) -> torch.Tensor | None:
+    """A decoder layer of a paged step of few rows in one host call (mllm_decoder_layer), or None when it does not apply:
+    another cache or backend, hooks, or operands its checks would refuse.  `layer` has passed `_small_ok`; the launches
+    are those of the submodules one after the other."""
+    if type(kv_cache) is not PagedStep or type(kv_cache.cache) is not PagedKVCache or x.dim() != 3 or x.shape[0] != 1:
+        return None
+    attn, norm1, norm2 = layer.self_attn, layer.input_layernorm, layer.post_attention_layernorm
+    backend, cfg, cache, meta = attn.backend, attn.config, kv_cache.cache, kv_cache.meta
+    if type(backend) is not HipBackend or not backend.fuse_rotary or backend.overlap_mixed \
+            or not _BACKEND_CALLS.isdisjoint(backend.__dict__):
+        return None
+    n, d = x.shape[1], x.shape[2]
+    h, hkv, dh = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+    wq, wk, wv = attn.q_proj, attn.k_proj, attn.v_proj
+    if not (bare(norm1, type(norm2)) and norm_ok(x, norm1.weight) and weights_ok(x, d, wq, wk, wv)
+            and weights_ok(x, h * dh, attn.o_proj)):
+        return None
+    wq, wk, wv = wq.weight, wk.weight, wv.weight
+    if wq.shape[0] != h * dh or wk.shape[0] != hkv * dh or wv.shape[0] != hkv * dh:
+        return None
+    if cos.shape != (1, n, dh) or sin.shape != cos.shape or not (_rows_ok(cos, x) and _rows_ok(sin, x)):
+        return None
+    i = attn.layer_idx
+    kc, vc = cache.k[i], cache.v[i]
+    if not (kc.dim() == 4 and kc.shape == vc.shape and kc.dtype == vc.dtype and kc.device == vc.device == x.device
+            and kc.shape[2] == hkv and kc.shape[3] == dh and kc.shape[1] == meta.block_size and kc.is_contiguous()
+            and vc.is_contiguous() and n == meta.query_start_loc[-1]):
+        return None
+    ks, vs = (cache.k_scale[i], cache.v_scale[i]) if cache.quantized else (1.0, 1.0)
+    if kc.dtype == FP8:
+        if not (0 < ks < math.inf and 0 < vs < math.inf):
+            return None
+    elif kc.dtype != x.dtype or ks != 1.0 or vs != 1.0:
+        return None
+    lib, mlp = _native.lib(), layer.mlp
+    gate = mlp.gate_proj.weight
+    ffn = gate.shape[0]
+    scratch = torch.empty(lib.fn("mllm_decoder_layer_scratch_bytes")(n, d, ffn, h, hkv, dh), dtype=torch.uint8,
+                          device=x.device)
+    step = backend.layer_step(meta, n, h, x.dtype, kc)
+    out = torch.empty_like(x)
+    lib.call("mllm_decoder_layer", step, x.data_ptr(), d, norm1.weight.data_ptr(), norm1.eps, wq.data_ptr(), wk.data_ptr(),
+             wv.data_ptr(), attn.o_proj.weight.data_ptr(), norm2.weight.data_ptr(), norm2.eps, gate.data_ptr(),
+             mlp.up_proj.weight.data_ptr(), mlp.down_proj.weight.data_ptr(), ffn, cos.data_ptr(), sin.data_ptr(),
+             dh, kc.data_ptr(), vc.data_ptr(), ks, vs, scratch.data_ptr(), scratch.numel(), out.data_ptr(),
+             _native.stream_ptr(x.device))
     return out

@@ -141,6 +141,9 @@ class LlamaDecoderLayer(nn.Module):
         fused = kernels.usable(x) and kernels.bare(norm, RMSNorm) and kernels.norm_ok(x, norm.weight)
         if fused and kernels.small_rows(x) and self._small_ok(x):
             attn, mlp = self.self_attn, self.mlp
+            out = kernels.decoder_layer(self, x, cos, sin, kv_cache)
+            if out is not None:
+                return out
             out = attn.attend(self.input_layernorm(x), cos, sin, kv_cache, key_valid)
             if kernels.small_rows(out) and kernels.weights_ok(out, out.shape[-1], attn.o_proj):
                 x, h = kernels.linear_add_norm(out, attn.o_proj.weight, x, norm.weight, norm.eps)

@@ -151,3 +151,48 @@ def test_decoder_layer_with_a_hook_calls_it(hip, part):
     assert seen == [1]
     # the two paths round at different places: a few bf16 roundings of values of some units
     torch.testing.assert_close(plain.float(), hooked.float(), rtol=4 * EPS[torch.bfloat16], atol=0.03)
+
+
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, None), (torch.bfloat16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("rows", [[(0, 1)], [(5, 1), (300, 1), (47, 1)], [(9, 1), (33, 20), (0, 40), (100, 2)], [(7, 1)] * 64,
+                                  [(3, 65)]])
+def test_decoder_layer_in_one_call(hip, dtype, kv, rows):
+    # the same launches as the submodules one after the other (which a backend with overlap_mixed set gets), bit for
+    # bit, on the output and both pools; more than 64 rows never take the call
+    from minillm.attention import get_backend
+    from minillm.attention.metadata import AttentionMetadata, SeqStep
+    from minillm.cache.paged import PagedKVCache
+    from minillm.model import kernels
+    from minillm.model.config import LlamaConfig
+    from minillm.model.llama import LlamaDecoderLayer
+
+    cfg = LlamaConfig(vocab_size=64, hidden_size=1024, intermediate_size=1536, num_hidden_layers=1, num_attention_heads=8,
+                      num_key_value_heads=2, head_dim=128, rms_norm_eps=1e-5, rope_theta=1e4, rope_scaling=None,
+                      max_position_embeddings=512)
+    backend = get_backend("hip")
+    torch.manual_seed(19)
+    layer = LlamaDecoderLayer(cfg, backend, 0).to(DEV, dtype)
+    n = sum(new for _, new in rows)
+    x, ang = _randn((1, n, 1024), dtype, 20), torch.randn(1, n, 128, device=DEV)
+    at, seqs = 0, []
+    for cached, new in rows:
+        need = -(-(cached + new) // 16)
+        seqs.append(SeqStep(cached, new, list(range(at, at + need))))
+        at += need
+    scales = {"k_scale": 0.02, "v_scale": 0.03} if kv else {}
+    results = []
+    with torch.inference_mode():
+        cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+        for overlap in (False, True):
+            backend.overlap_mixed = overlap
+            g = torch.Generator(device=DEV).manual_seed(21)
+            cache = PagedKVCache(cfg, at, DEV, kv or dtype, **scales)
+            for pool in (cache.k[0], cache.v[0]):
+                pool.copy_(torch.randn(pool.shape, device=DEV, generator=g).to(pool.dtype))
+            step = cache.step(AttentionMetadata.build(seqs, 16, DEV))
+            assert kernels.small_rows(x) == (n <= 64)
+            if n <= 64:
+                assert (kernels.decoder_layer(layer, x, cos, sin, step) is None) == overlap
+            results.append((layer(x, cos, sin, step), cache.k[0], cache.v[0]))
+    for a, b in zip(*results):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
