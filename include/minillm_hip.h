@@ -317,6 +317,11 @@ int mllm_rms_norm(const void* x, const void* residual, const void* weight, int64
  * 8, pointers 16-byte aligned. */
 int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_t dtype, void* out, void* stream);
 
+/* Rotary tables (reference src/minillm/model/llama.py:51-56): cos / sin [n, 2 half] = T(cos / sin(float(positions[t]) *
+ * inv_freq[d % half])), fp32 angles, T the 16-bit `dtype`. */
+int mllm_rope_table(const int64_t* positions, int64_t n, const float* inv_freq, int32_t half, int32_t dtype, void* cos,
+                    void* sin, void* stream);
+
 /*
  * Linear layers of few rows (reference src/minillm/model/llama.py:75-120): x [m, k] contiguous, weights [n, k] contiguous
  * as torch.nn.Linear holds them, m <= 64, k a multiple of 256, n multiples of 16, BF16 or F16, fp32 sums, 16-byte

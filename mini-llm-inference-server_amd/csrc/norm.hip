@@ -146,6 +146,24 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restri
   st16(out + i, pack8<T>(f));
 }
 
+// cos and sin rows of the rotary embedding: out[t][d] = T(cos(float(pos[t]) * inv_freq[d % half])), one thread per
+// frequency and both of its places.  Bound by the launch: as seven elementwise launches a step's rows took 25 us.
+template <typename T>
+__global__ __launch_bounds__(256) void rope_table_kernel(const int64_t* __restrict__ pos, int64_t n,
+                                                         const float* __restrict__ inv_freq, int half,
+                                                         uint16_t* __restrict__ cos_out,
+                                                         uint16_t* __restrict__ sin_out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n * half) return;
+  const int64_t t = i / half;
+  const int d = (int)(i - t * half);
+  const float ang = (float)pos[t] * inv_freq[d];
+  const uint16_t c = cvt1<T>(cosf(ang)), s = cvt1<T>(sinf(ang));
+  const int64_t o = 2 * t * half + d;
+  cos_out[o] = cos_out[o + half] = c;
+  sin_out[o] = sin_out[o + half] = s;
+}
+
 }  // namespace
 }  // namespace mllm
 
@@ -239,4 +257,22 @@ extern "C" int mllm_sum_partials_norm(const float* part, int32_t ksplit, const v
   else
     launch(F16{});
   return check_launch("mllm_sum_partials_norm");
+}
+
+extern "C" int mllm_rope_table(const int64_t* positions, int64_t n, const float* inv_freq, int32_t half, int32_t dtype,
+                               void* cos, void* sin, void* stream) {
+  using namespace mllm;
+  MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
+               "mllm_rope_table: dtype must be bfloat16 or float16");
+  MLLM_REQUIRE(n >= 0 && half > 0 && n < (1ll << 31), MLLM_ERR_INVALID, "mllm_rope_table: bad sizes");
+  if (n == 0) return MLLM_OK;
+  MLLM_REQUIRE(positions && inv_freq && cos && sin, MLLM_ERR_INVALID, "mllm_rope_table: null pointer");
+  const int64_t groups = (n * half + 255) / 256;
+  MLLM_REQUIRE(groups < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_rope_table: too many positions");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (dtype == MLLM_DTYPE_BF16)
+    rope_table_kernel<BF16><<<(unsigned)groups, 256, 0, st>>>(positions, n, inv_freq, half, (uint16_t*)cos, (uint16_t*)sin);
+  else
+    rope_table_kernel<F16><<<(unsigned)groups, 256, 0, st>>>(positions, n, inv_freq, half, (uint16_t*)cos, (uint16_t*)sin);
+  return check_launch("mllm_rope_table");
 }

@@ -70,6 +70,7 @@ SIGNATURES = {
     "mllm_sum_partials": (ctypes.c_int, [_p, _i32, _i64, _i64, _p, _i32, _p, _p]),
     "mllm_sum_partials_norm": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
     "mllm_linear_swiglu": (ctypes.c_int, [_p, _i64, _i64, _p, _p, _i64, _i32, _p, _p]),
+    "mllm_rope_table": (ctypes.c_int, [_p, _i64, _p, _i32, _i32, _p, _p, _p]),
     "mllm_linear_ksplit": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
     "mllm_decoder_layer_scratch_bytes": (ctypes.c_int64, [_i64, _i64, _i64, _i32, _i32, _i32]),
     "mllm_decoder_layer": (ctypes.c_int, [_p, _p, _i64, _p, _f32, _p, _p, _p, _p, _p, _f32, _p, _p, _p, _i64, _p, _p, _i64,

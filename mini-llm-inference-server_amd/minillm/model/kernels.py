@@ -25,8 +25,9 @@ _BACKEND_CALLS = frozenset(("forward", "forward_rotary", "run_layer", "rope_appe
 _wrapped = torch._C._functorch.is_functorch_wrapped_tensor
 
 
-def usable(x: torch.Tensor) -> bool:
-    return (type(x) is torch.Tensor and x.is_cuda and x.dtype in _DTYPES and not torch.is_grad_enabled()
+def usable(x: torch.Tensor, dtype: torch.dtype | None = None) -> bool:
+    """`dtype`: the type of the call's operands where x is not one of them."""
+    return (type(x) is torch.Tensor and x.is_cuda and (dtype or x.dtype) in _DTYPES and not torch.is_grad_enabled()
             and not torch.is_autocast_enabled() and not torch._C._len_torch_dispatch_stack()
             and not torch._C._len_torch_function_stack() and not _wrapped(x) and forward_ad._current_level < 0
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
@@ -71,6 +72,16 @@ def add_rms_norm(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: fl
     _native.lib().call("mllm_rms_norm", x.data_ptr(), y.data_ptr(), weight.data_ptr(), x.numel() // d, d, eps,
                        _native.dtype_code(x.dtype), total.data_ptr(), out.data_ptr(), _native.stream_ptr(x.device))
     return total, out
+
+
+def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype):
+    """cos, sin [..., 2 len(inv_freq)] of int64 positions."""
+    half = inv_freq.shape[0]
+    cos = torch.empty((*positions.shape, 2 * half), dtype=dtype, device=positions.device)
+    sin = torch.empty_like(cos)
+    _native.lib().call("mllm_rope_table", positions.data_ptr(), positions.numel(), inv_freq.data_ptr(), half,
+                       _native.dtype_code(dtype), cos.data_ptr(), sin.data_ptr(), _native.stream_ptr(positions.device))
+    return cos, sin
 
 
 def sum_ok(x: torch.Tensor, y: torch.Tensor) -> bool:

@@ -48,6 +48,24 @@ def test_silu_mul(hip, dtype, n):
     torch.testing.assert_close(out.double(), g / (1 + torch.exp(-g)) * up.double(), rtol=1.01 * EPS[dtype], atol=1e-7)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 1), (2, 37), (1, 1000)])
+def test_rope_table(hip, dtype, shape):
+    from minillm.model.config import LLAMA_3_1_8B, LlamaConfig
+    from minillm.model.llama import RotaryEmbedding
+
+    rot = RotaryEmbedding(LlamaConfig(**LLAMA_3_1_8B))
+    pos = torch.randint(0, 131072, shape, generator=torch.Generator().manual_seed(22)).to(DEV)
+    pos[0, 0] = 0
+    with torch.no_grad():
+        got = rot(pos, dtype)
+    exp = rot(pos, dtype)  # gradients on: torch's expressions
+    # the same fp32 angles; cos and sin within some 2^-24 before one rounding, which may then fall to the other side
+    for g, e in zip(got, exp):
+        assert g.shape == (*shape, 128) and g.dtype == dtype
+        torch.testing.assert_close(g.float(), e.float(), rtol=2 * EPS[dtype], atol=1e-6)
+
+
 def test_torch_path_kept(hip):
     # gradients, hooks, float32, odd widths and transforms see torch's own operations
     from minillm.model import kernels
