@@ -92,8 +92,9 @@ class AttentionMetadata:
         n_tok = starts[-1]
         n_pages = sum(-(-n // bs) for n in lens)
 
-        host = pack_steps(seqs, np.empty(3 * n_seq + 1 + n_ids, dtype=np.int32))
-        packed = torch.from_numpy(host).to(device)
+        staged = _staging(3 * n_seq + 1 + n_ids)
+        pack_steps(seqs, staged.numpy())
+        packed = staged.to(device, non_blocking=True)
         meta = cls._arenas(bs, starts, lens, n_tok, width, n_pages, device)
         meta._launch_build(packed, width)
         meta._upload = packed  # keeps the input alive until the launches that read it have run
@@ -208,13 +209,14 @@ class DeviceBlockTables:
         rows, updates = self.sync(keys, seqs)
         n_seq = len(seqs)
         nblk = [len(s.block_ids) for s in seqs]
-        host = np.empty(4 * n_seq + len(updates), dtype=np.int32)
+        staged = _staging(4 * n_seq + len(updates))
+        host = staged.numpy()
         host[:n_seq] = [s.num_cached for s in seqs]
         host[n_seq:2 * n_seq] = [s.num_new for s in seqs]
         host[2 * n_seq:3 * n_seq] = rows
         host[3 * n_seq:4 * n_seq] = nblk
         host[4 * n_seq:] = updates
-        packed = torch.from_numpy(host).to(self.device)
+        packed = staged.to(self.device, non_blocking=True)
         width = max(nblk)
         meta = AttentionMetadata._arenas(bs, starts, lens, starts[-1], width, sum(-(-n // bs) for n in lens),
                                          self.device)
@@ -228,6 +230,13 @@ class DeviceBlockTables:
         if num_updates:
             _native.lib().call("mllm_update_block_tables", self.tables.data_ptr(), self.tables.numel(),
                                packed.data_ptr() + 4 * offset, num_updates, _native.stream_ptr(self.device))
+
+
+def _staging(n: int) -> torch.Tensor:
+    """Pinned int32 memory for one upload.  A copy out of pageable memory returns only when the stream has reached it,
+    so each step waited for the one before (decode steps of 32 rows 623 against 511 us); out of pinned memory it is
+    enqueued, and torch's host allocator gives the block to a later step only once the copy has run."""
+    return torch.empty(n, dtype=torch.int32, pin_memory=True)
 
 
 def pack_steps(seqs: list[SeqStep], out: np.ndarray) -> np.ndarray:
