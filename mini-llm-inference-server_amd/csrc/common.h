@@ -23,6 +23,11 @@ int check_launch(const char* what);
     if (!(cond)) return ::mllm::fail((code), (msg)); \
   } while (0)
 
+// Decode of the rows with one new token among the step's first `rows` sequences by row workgroups
+// (decode_rows_kernel): q as given, out [N, H, Dh].
+int paged_decode_rows(const mllm_layer_step& s, const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                      const void* k_cache, const void* v_cache, int32_t rows, void* out, void* stream);
+
 // ---------------------------------------------------------------- types
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
