@@ -115,14 +115,14 @@ def small_rows(x: torch.Tensor) -> bool:
 
 def weights_ok(like: torch.Tensor, k: int, *linears) -> bool:
     """Whether the few-row kernels take these layers for operands of `k` columns with the type and device of `like`."""
-    if k % CHUNK:
+    if k % CHUNK or k >= 1 << 24:
         return False
     for m in linears:
         params = m.__dict__["_parameters"]
         if not bare(m, torch.nn.Linear) or params["bias"] is not None:
             return False
         w = params["weight"]
-        if w.shape[1] != k or w.shape[0] % 16 or not _plain_weight(w, like):
+        if w.shape[1] != k or w.shape[0] % 16 or w.shape[0] >= 1 << 28 or not _plain_weight(w, like):
             return False
     return True
 
