@@ -177,11 +177,11 @@ def row_workgroups(num_new: list[int], seq_lens: list[int], num_heads: int, num_
     500 tokens 32 rows 18.4 against 20.9 us, 8 rows 15.4 against 13.5 with one launch less for the host (4 rows of
     37-500 tokens, called eagerly: 19.9 against 22.1 us); 48 rows 27.9 against 26.8.  8 rows of 200-1,000 tokens:
     21.8 against 15.3 us.  16-bit pools (the fp8 kernels keep bins); a forced bin size keeps bins."""
-    if kv_fp8 or head_dim != 128 or os.environ.get("MLLM_PAGES_PER_SPLIT"):
-        return 0
     groups = len(seq_lens) * num_kv_heads
+    if groups > ROW_GROUPS or kv_fp8 or head_dim != 128 or os.environ.get("MLLM_PAGES_PER_SPLIT"):
+        return 0
     longest = max((n for n, new in zip(seq_lens, num_new) if new == 1), default=0)
-    if not longest or groups > ROW_GROUPS or longest > (ROW_TOKENS_ALONE if groups <= FULL_CHIP_CUS else ROW_TOKENS):
+    if not longest or longest > (ROW_TOKENS_ALONE if groups <= FULL_CHIP_CUS else ROW_TOKENS):
         return 0
     return len(seq_lens)
 
