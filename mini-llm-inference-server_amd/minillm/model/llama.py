@@ -6,7 +6,8 @@ The hot path's call site is `LlamaAttention.forward` on a ragged paged step: q/k
 go to `backend.forward(q[N,H,Dh], k[N,Hkv,Dh], v[N,Hkv,Dh], k_pool[layer], v_pool[layer], meta)`,
 which appends k/v to the pool and returns the attention output.  Where `kernels.usable` allows it (16-bit
 tensors, no gradients) RMSNorm, the residual sum before it and SwiGLU run as one kernel each, and the
-products of steps of up to 64 rows as few-row kernels; everything else stays in PyTorch.  Without a cache (kv_cache None) the contiguous `backend.prefill` path runs instead.
+products of steps of up to 64 rows as few-row kernels; everything else stays in PyTorch.  Without a cache
+(kv_cache None) the contiguous `backend.prefill` path runs instead.
 """
 
 from __future__ import annotations
@@ -172,7 +173,7 @@ class LlamaDecoderLayer(nn.Module):
         if not (kernels.weights_ok(x, d, gate, up) and gate.weight.shape == up.weight.shape):
             return False
         return kernels.weights_ok(x, gate.weight.shape[0], down) and down.weight.shape[0] == d \
-            and attn.o_proj.weight.shape[0] == d
+            and kernels.bare(attn.o_proj, nn.Linear) and attn.o_proj.weight.shape[0] == d
 
 
 class LlamaModel(nn.Module):

@@ -171,6 +171,38 @@ def test_decoder_layer_with_a_hook_calls_it(hip, part):
     torch.testing.assert_close(plain.float(), hooked.float(), rtol=4 * EPS[torch.bfloat16], atol=0.03)
 
 
+@pytest.mark.parametrize("where", ["self_attn.q_proj", "self_attn.o_proj", "mlp.up_proj", "mlp.down_proj", "mlp",
+                                   "input_layernorm", "post_attention_layernorm"])
+def test_decoder_layer_with_a_wrapped_submodule(hip, where):
+    # a submodule that is not the plain class and has no weight of its own (an adapter, a quantized layer) is called
+    from minillm.attention import get_backend
+    from minillm.model.config import LlamaConfig
+    from minillm.model.llama import LlamaDecoderLayer
+
+    class Wrap(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return self.inner(x)
+
+    cfg = LlamaConfig(vocab_size=64, hidden_size=512, intermediate_size=768, num_hidden_layers=1, num_attention_heads=4,
+                      num_key_value_heads=2, head_dim=128, rms_norm_eps=1e-5, rope_theta=1e4)
+    torch.manual_seed(24)
+    layer = LlamaDecoderLayer(cfg, get_backend("hip"), 0).to(DEV, torch.bfloat16)
+    x, ang = _randn((1, 9, 512), torch.bfloat16, 25), torch.randn(1, 9, 128, device=DEV)
+    with torch.inference_mode():
+        cos, sin = ang.cos().bfloat16(), ang.sin().bfloat16()
+        plain = layer(x, cos, sin)
+        parent = layer.get_submodule(where.rpartition(".")[0])
+        name = where.rpartition(".")[2]
+        setattr(parent, name, Wrap(getattr(parent, name)))
+        wrapped = layer(x, cos, sin)
+    # the two paths round at different places: a few bf16 roundings of values of some units
+    torch.testing.assert_close(plain.float(), wrapped.float(), rtol=4 * EPS[torch.bfloat16], atol=0.03)
+
+
 @pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, None), (torch.bfloat16, torch.float8_e4m3fn)])
 @pytest.mark.parametrize("rows", [[(0, 1)], [(5, 1), (300, 1), (47, 1)], [(9, 1), (33, 20), (0, 40), (100, 2)], [(7, 1)] * 64,
                                   [(3, 65)]])
