@@ -26,11 +26,12 @@ _wrapped = torch._C._functorch.is_functorch_wrapped_tensor
 
 
 def usable(x: torch.Tensor, dtype: torch.dtype | None = None) -> bool:
-    """`dtype`: the type of the call's operands where x is not one of them."""
-    return (type(x) is torch.Tensor and x.is_cuda and (dtype or x.dtype) in _DTYPES and not torch.is_grad_enabled()
-            and not torch.is_autocast_enabled() and not torch._C._len_torch_dispatch_stack()
-            and not torch._C._len_torch_function_stack() and not _wrapped(x) and forward_ad._current_level < 0
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+    """`dtype`: the type of the call's operands where x is not one of them.  Whether a compiler is at work is asked first:
+    dynamo knows that answer while it traces and leaves out the rest, some of which it cannot trace."""
+    return (not torch.compiler.is_compiling() and type(x) is torch.Tensor and x.is_cuda
+            and (dtype or x.dtype) in _DTYPES and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and not torch._C._len_torch_dispatch_stack() and not torch._C._len_torch_function_stack()
+            and not _wrapped(x) and forward_ad._current_level < 0 and not torch.jit.is_tracing()
             and x.device.index == torch.cuda.current_device() and _native.available())
 
 

@@ -88,6 +88,25 @@ def test_torch_path_kept(hip):
     assert not kernels.bare(norm, RMSNorm)
 
 
+@pytest.mark.parametrize("part", ["norm", "mlp", "rotary"])
+def test_modules_compile_as_one_graph(hip, part):
+    from minillm.model import llama
+    from minillm.model.config import LlamaConfig
+
+    cfg = LlamaConfig(vocab_size=64, hidden_size=512, intermediate_size=768, num_hidden_layers=1, num_attention_heads=4,
+                      num_key_value_heads=2, head_dim=128, rms_norm_eps=1e-5, rope_theta=1e4)
+    x = _randn((1, 3, 512), torch.bfloat16, 26)
+    module, args = {"norm": (llama.RMSNorm(512, 1e-5), (x,)), "mlp": (llama.LlamaMLP(cfg), (x,)),
+                    "rotary": (llama.RotaryEmbedding(cfg), (torch.arange(3, device=DEV)[None], torch.bfloat16))}[part]
+    module = module.to(DEV, torch.bfloat16)
+    with torch.no_grad():
+        compiled = torch.compile(module, fullgraph=True, backend="eager")
+        got_exp = compiled(*args), module(*args)
+    # the kernels keep silu and the norm in fp32 where torch's expressions round: a few bf16 roundings of values below 4
+    for got, exp in zip(*(y if part == "rotary" else (y,) for y in got_exp)):
+        torch.testing.assert_close(got.float(), exp.float(), rtol=4 * EPS[torch.bfloat16], atol=0.03)
+
+
 def _ref(x, w):
     return x.double() @ w.double().t()
 
