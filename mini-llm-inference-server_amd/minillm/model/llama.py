@@ -30,8 +30,9 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x * rsqrt(mean(x^2) + eps) computed in float32, cast back, then scaled by the weight."""
-        if kernels.usable(x) and kernels.norm_ok(x, self.weight):
-            return kernels.rms_norm(x, self.weight, self.eps)
+        if not torch.jit.is_scripting():  # a scripted module keeps the torch expressions
+            if kernels.usable(x) and kernels.norm_ok(x, self.weight):
+                return kernels.rms_norm(x, self.weight, self.eps)
         h = x.float()
         h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + self.eps)
         return self.weight * h.to(x.dtype)
@@ -129,7 +130,10 @@ class LlamaMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         gate, up = self.gate_proj(x), self.up_proj(x)
-        return self.down_proj(kernels.silu_mul(gate, up) if kernels.silu_mul_ok(gate, up) else F.silu(gate) * up)
+        if not torch.jit.is_scripting():
+            if kernels.silu_mul_ok(gate, up):
+                return self.down_proj(kernels.silu_mul(gate, up))
+        return self.down_proj(F.silu(gate) * up)
 
 
 class LlamaDecoderLayer(nn.Module):

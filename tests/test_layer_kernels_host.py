@@ -1,0 +1,17 @@
+"""Which calls keep torch's expressions instead of the decoder layer's kernels, as far as that shows without a GPU."""
+
+import pytest
+import torch
+
+from minillm.model import llama
+from minillm.model.config import LlamaConfig
+
+CFG = LlamaConfig(vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1, num_attention_heads=4,
+                  num_key_value_heads=2, head_dim=16, rms_norm_eps=1e-5, rope_theta=1e4)
+
+
+@pytest.mark.parametrize("module", [llama.RMSNorm(64, 1e-5), llama.LlamaMLP(CFG)], ids=["norm", "mlp"])
+def test_modules_can_be_scripted(module):
+    x = torch.randn(3, 64, generator=torch.Generator().manual_seed(0))
+    with torch.no_grad():
+        assert torch.equal(torch.jit.script(module)(x), module(x))
