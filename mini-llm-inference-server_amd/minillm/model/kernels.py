@@ -22,16 +22,18 @@ from ..cache.paged import PagedKVCache, PagedStep
 _DTYPES = (torch.bfloat16, torch.float16)
 # what mllm_decoder_layer stands in for: a backend instance that overrides one of these is called instead
 _BACKEND_CALLS = frozenset(("forward", "forward_rotary", "run_layer", "rope_append", "append", "attend"))
-_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_transform = torch._C._functorch.peek_interpreter_stack  # the innermost active functorch transform, or None
+_wrapped = torch._C._functorch.is_functorch_wrapped_tensor  # also of a wrapper that outlived its transform
 
 
 def usable(x: torch.Tensor, dtype: torch.dtype | None = None) -> bool:
     """`dtype`: the type of the call's operands where x is not one of them.  Whether a compiler is at work is asked first:
-    dynamo knows that answer while it traces and leaves out the rest, some of which it cannot trace."""
+    dynamo knows that answer while it traces and leaves out the rest, some of which it cannot trace.  Inside a transform
+    (vmap and the like) any operand may be a wrapper without storage, not only x, so none is let through."""
     return (not torch.compiler.is_compiling() and type(x) is torch.Tensor and x.is_cuda
             and (dtype or x.dtype) in _DTYPES and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
             and not torch._C._len_torch_dispatch_stack() and not torch._C._len_torch_function_stack()
-            and not _wrapped(x) and forward_ad._current_level < 0 and not torch.jit.is_tracing()
+            and _transform() is None and not _wrapped(x) and forward_ad._current_level < 0 and not torch.jit.is_tracing()
             and x.device.index == torch.cuda.current_device() and _native.available())
 
 
@@ -44,8 +46,9 @@ def bare(module: torch.nn.Module, cls: type) -> bool:
 
 
 def _rows_ok(t: torch.Tensor, like: torch.Tensor) -> bool:
-    """A contiguous, 16-byte aligned operand of the same type and device."""
-    return t.dtype == like.dtype and t.device == like.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+    """A contiguous, 16-byte aligned operand of the same type and device, with storage."""
+    return not _wrapped(t) and t.dtype == like.dtype and t.device == like.device and t.is_contiguous() \
+        and t.data_ptr() % 16 == 0
 
 
 def _plain_weight(w, like: torch.Tensor) -> bool:

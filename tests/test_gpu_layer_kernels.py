@@ -88,6 +88,28 @@ def test_torch_path_kept(hip):
     assert not kernels.bare(norm, RMSNorm)
 
 
+@pytest.mark.parametrize("part", ["norm", "mlp"])
+def test_vmap_over_weights(hip, part):
+    # an ensemble: one x, a batch of parameters
+    from minillm.model import llama
+    from minillm.model.config import LlamaConfig
+
+    cfg = LlamaConfig(vocab_size=64, hidden_size=512, intermediate_size=768, num_hidden_layers=1, num_attention_heads=4,
+                      num_key_value_heads=2, head_dim=128, rms_norm_eps=1e-5, rope_theta=1e4)
+    x = _randn((3, 512), torch.bfloat16, 27)
+    modules = [(llama.RMSNorm(512, 1e-5) if part == "norm" else llama.LlamaMLP(cfg)).to(DEV, torch.bfloat16)
+               for _ in range(2)]
+    with torch.no_grad():
+        for i, m in enumerate(modules):
+            for p in m.parameters():
+                p.add_(0.01 * i)
+        params, _ = torch.func.stack_module_state(modules)
+        got = torch.func.vmap(lambda p: torch.func.functional_call(modules[0], p, (x,)))(params)
+        exp = torch.stack([m(x) for m in modules])
+    # torch's expressions against the kernels: a few bf16 roundings of values below 4
+    torch.testing.assert_close(got.float(), exp.float(), rtol=4 * EPS[torch.bfloat16], atol=0.03)
+
+
 @pytest.mark.parametrize("part", ["norm", "mlp", "rotary"])
 def test_modules_compile_as_one_graph(hip, part):
     from minillm.model import llama

@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from minillm.model import llama
+from minillm.model import kernels, llama
 from minillm.model.config import LlamaConfig
 
 CFG = LlamaConfig(vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1, num_attention_heads=4,
@@ -15,3 +15,19 @@ def test_modules_can_be_scripted(module):
     x = torch.randn(3, 64, generator=torch.Generator().manual_seed(0))
     with torch.no_grad():
         assert torch.equal(torch.jit.script(module)(x), module(x))
+
+
+def test_wrapped_operands_are_refused():
+    # tensors of a functorch transform, while it runs and after it: no storage to hand to a kernel
+    x, seen = torch.zeros(3, 64, dtype=torch.bfloat16), []
+
+    def look(t):
+        seen.append(t)
+        assert not kernels.sum_ok(x, t) and not kernels.norm_ok(x, t) and not kernels.small_rows(t)
+        return t.sum()
+
+    torch.func.vmap(look)(torch.zeros(2, 64, dtype=torch.bfloat16))
+    torch.func.grad(look)(torch.zeros(64, dtype=torch.bfloat16))
+    for t in seen:
+        assert not kernels.norm_ok(x, t)
+    assert kernels.norm_ok(x, torch.zeros(64, dtype=torch.bfloat16))
