@@ -122,8 +122,10 @@ def weights_ok(like: torch.Tensor, k: int, *linears) -> bool:
     if k % CHUNK or k >= 1 << 24:
         return False
     for m in linears:
+        # taken from the registered parameters; a layer that holds them as plain attributes (a data-parallel replica)
+        # is called
         params = m.__dict__["_parameters"]
-        if not bare(m, torch.nn.Linear) or params["bias"] is not None:
+        if not bare(m, torch.nn.Linear) or params.get("bias", m) is not None or params.get("weight") is None:
             return False
         w = params["weight"]
         if w.shape[1] != k or w.shape[0] % 16 or w.shape[0] >= 1 << 28 or not _plain_weight(w, like):

@@ -31,3 +31,18 @@ def test_wrapped_operands_are_refused():
     for t in seen:
         assert not kernels.norm_ok(x, t)
     assert kernels.norm_ok(x, torch.zeros(64, dtype=torch.bfloat16))
+
+
+def test_weights_held_as_plain_attributes():
+    x = torch.zeros(3, 256, dtype=torch.bfloat16)
+    lin = torch.nn.Linear(256, 32, bias=False, dtype=torch.bfloat16)
+    assert kernels.weights_ok(x, 256, lin)
+    replica = lin._replicate_for_data_parallel()
+    replica.weight, replica.bias = lin.weight.detach(), None
+    assert not kernels.weights_ok(x, 256, replica)
+    for name in ("weight", "bias"):
+        other = torch.nn.Linear(256, 32, bias=name == "bias", dtype=torch.bfloat16)
+        value = getattr(other, name).detach()
+        delattr(other, name)
+        setattr(other, name, value)
+        assert not kernels.weights_ok(x, 256, other)
