@@ -23,6 +23,9 @@ int check_launch(const char* what);
     if (!(cond)) return ::mllm::fail((code), (msg)); \
   } while (0)
 
+// HIP takes fewer than 2^32 work-items along x: workgroups of 256 threads a launch may have.
+constexpr int64_t kMaxGroups256 = (1ll << 24) - 1;
+
 // Decode of the rows with one new token among the step's first `rows` sequences by row workgroups
 // (decode_rows_kernel): q as given, out [N, H, Dh].
 int paged_decode_rows(const mllm_layer_step& s, const void* q, int64_t q_stride_tok, int64_t q_stride_head,

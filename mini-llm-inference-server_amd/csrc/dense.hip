@@ -975,14 +975,15 @@ bool mfma_operands(const DenseArgs& a, int per16) {
 // 34.6 us, 800 (four of 777) 42.5 against 65.1 us.  A workgroup of 32 rows reads four times the K and V per row.
 constexpr int64_t kLargeMin = 384;
 
+// Workgroups of `rows` query rows.
+int64_t items(const DenseArgs& a, int rows) {
+  const int tokens = rows / a.G;
+  return (int64_t)((a.Tq + tokens - 1) / tokens) * a.B * (a.H / a.G);
+}
+
 template <typename T, int DH>
 int launch_mfma(const DenseArgs& a, hipStream_t st) {
-  const auto items = [&](int rows) {
-    const int tokens = rows / a.G;
-    return (int64_t)((a.Tq + tokens - 1) / tokens) * a.B * (a.H / a.G);
-  };
-  const int64_t large = items(128), small = items(32);
-  MLLM_REQUIRE(small < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_dense_attention: grid too large");
+  const int64_t large = items(a, 128), small = items(a, 32);
   if (large >= kLargeMin) {
     if (a.key_valid)
       dense_mfma_kernel<T, DH, true><<<(unsigned)large, 256, 0, st>>>(a);
@@ -998,18 +999,16 @@ int launch_mfma(const DenseArgs& a, hipStream_t st) {
 }
 
 int launch_f32(const DenseArgs& a, hipStream_t st) {
-  const int tokens = 16 / a.G;
-  const int64_t items = (int64_t)((a.Tq + tokens - 1) / tokens) * a.B * (a.H / a.G);
-  MLLM_REQUIRE(items < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_dense_attention: grid too large");
+  const unsigned groups = (unsigned)items(a, 16);
   if (a.Dh == 128) {
     if (a.key_valid)
-      dense_f32_kernel<128, true><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+      dense_f32_kernel<128, true><<<groups, 64 * kWavesF32, 0, st>>>(a);
     else
-      dense_f32_kernel<128, false><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+      dense_f32_kernel<128, false><<<groups, 64 * kWavesF32, 0, st>>>(a);
   } else if (a.key_valid) {
-    dense_f32_kernel<64, true><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+    dense_f32_kernel<64, true><<<groups, 64 * kWavesF32, 0, st>>>(a);
   } else {
-    dense_f32_kernel<64, false><<<(unsigned)items, 64 * kWavesF32, 0, st>>>(a);
+    dense_f32_kernel<64, false><<<groups, 64 * kWavesF32, 0, st>>>(a);
   }
   return check_launch("mllm_dense_attention");
 }
@@ -1040,11 +1039,12 @@ extern "C" int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, i
               kv_len, head_dim, pack, softmax_scale};
   dim3 grid(q_len, num_heads, batch);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // (more workgroups than a launch takes: dense_kernel, whose grid has the heads and the batch along y and z)
   if (dtype == MLLM_DTYPE_F32 && (head_dim == 128 || head_dim == 64) && mfma_operands(a, 4)) {
     a.G = 16 % group == 0 ? group : 1;
-    return launch_f32(a, st);
+    if (items(a, 16) <= kMaxGroups256) return launch_f32(a, st);
   }
-  if (dtype != MLLM_DTYPE_F32 && mfma_operands(a, 8)) {
+  if (dtype != MLLM_DTYPE_F32 && mfma_operands(a, 8) && items(a, 32) <= kMaxGroups256) {
     const bool bf16 = dtype == MLLM_DTYPE_BF16;
     if (head_dim == 128)
       return bf16 ? launch_mfma<BF16, 128>(a, st) : launch_mfma<F16, 128>(a, st);

@@ -209,7 +209,7 @@ extern "C" int mllm_linear_partial(const void* x, int64_t m, int64_t k, const vo
     cols += n[i];
   }
   MLLM_REQUIRE(n1 > 0 || n2 == 0, MLLM_ERR_INVALID, "mllm_linear_partial: weights are given from the first on");
-  MLLM_REQUIRE(tiles * ksplit < (1ll << 31) && cols < (1ll << 31), MLLM_ERR_UNSUPPORTED,
+  MLLM_REQUIRE(tiles * ksplit <= kMaxGroups256 / 2 && cols < (1ll << 31), MLLM_ERR_UNSUPPORTED,
                "mllm_linear_partial: too many tiles");
   if (m == 0) return MLLM_OK;
   MLLM_REQUIRE(part, MLLM_ERR_INVALID, "mllm_linear_partial: null pointer");

@@ -172,8 +172,9 @@ extern "C" int mllm_rms_norm(const void* x, const void* residual, const void* we
   using namespace mllm;
   MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
                "mllm_rms_norm: dtype must be bfloat16 or float16");
-  MLLM_REQUIRE(rows >= 0 && rows < (1ll << 31) && dim > 0 && dim % 8 == 0 && dim < (1ll << 31), MLLM_ERR_INVALID,
+  MLLM_REQUIRE(rows >= 0 && dim > 0 && dim % 8 == 0 && dim < (1ll << 31), MLLM_ERR_INVALID,
                "mllm_rms_norm: need rows >= 0 and a positive dim, a multiple of 8");
+  MLLM_REQUIRE(rows <= kMaxGroups256, MLLM_ERR_UNSUPPORTED, "mllm_rms_norm: fewer than 2^24 rows");
   MLLM_REQUIRE(!residual == !sum, MLLM_ERR_INVALID, "mllm_rms_norm: residual and sum go together");
   if (rows == 0) return MLLM_OK;
   MLLM_REQUIRE(x && weight && out, MLLM_ERR_INVALID, "mllm_rms_norm: null pointer");
@@ -199,7 +200,8 @@ extern "C" int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_
   using namespace mllm;
   MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
                "mllm_silu_mul: dtype must be bfloat16 or float16");
-  MLLM_REQUIRE(n >= 0 && n % 8 == 0 && n < (1ll << 38), MLLM_ERR_INVALID, "mllm_silu_mul: n must be a multiple of 8");
+  MLLM_REQUIRE(n >= 0 && n % 8 == 0, MLLM_ERR_INVALID, "mllm_silu_mul: n must be a multiple of 8");
+  MLLM_REQUIRE(n <= kMaxGroups256 * 2048, MLLM_ERR_UNSUPPORTED, "mllm_silu_mul: too many elements");
   if (n == 0) return MLLM_OK;
   MLLM_REQUIRE(gate && up && out, MLLM_ERR_INVALID, "mllm_silu_mul: null pointer");
   MLLM_REQUIRE(((uintptr_t)gate | (uintptr_t)up | (uintptr_t)out) % 16 == 0, MLLM_ERR_UNSUPPORTED,
@@ -225,7 +227,7 @@ extern "C" int mllm_sum_partials(const float* part, int32_t ksplit, int64_t rows
   MLLM_REQUIRE(((uintptr_t)part | (uintptr_t)residual | (uintptr_t)out) % 16 == 0, MLLM_ERR_UNSUPPORTED,
                "mllm_sum_partials: operands must be 16-byte aligned");
   const int64_t n = rows * dim, groups = (n / 8 + 255) / 256;
-  MLLM_REQUIRE(groups < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_sum_partials: too many elements");
+  MLLM_REQUIRE(groups <= kMaxGroups256, MLLM_ERR_UNSUPPORTED, "mllm_sum_partials: too many elements");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (dtype == MLLM_DTYPE_BF16)
     sum_partials_kernel<BF16><<<(unsigned)groups, 256, 0, st>>>(part, ksplit, n, (const uint16_t*)residual, (uint16_t*)out);
@@ -240,8 +242,9 @@ extern "C" int mllm_sum_partials_norm(const float* part, int32_t ksplit, const v
   using namespace mllm;
   MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
                "mllm_sum_partials_norm: dtype must be bfloat16 or float16");
-  MLLM_REQUIRE(ksplit >= 1 && rows >= 0 && dim > 0 && dim % 8 == 0 && rows < (1ll << 31) && dim < (1ll << 31),
-               MLLM_ERR_INVALID, "mllm_sum_partials_norm: bad sizes");
+  MLLM_REQUIRE(ksplit >= 1 && rows >= 0 && dim > 0 && dim % 8 == 0 && dim < (1ll << 31), MLLM_ERR_INVALID,
+               "mllm_sum_partials_norm: bad sizes");
+  MLLM_REQUIRE(rows <= kMaxGroups256, MLLM_ERR_UNSUPPORTED, "mllm_sum_partials_norm: fewer than 2^24 rows");
   if (rows == 0) return MLLM_OK;
   MLLM_REQUIRE(part && residual && weight && sum && out, MLLM_ERR_INVALID, "mllm_sum_partials_norm: null pointer");
   MLLM_REQUIRE(((uintptr_t)part | (uintptr_t)residual | (uintptr_t)weight | (uintptr_t)sum | (uintptr_t)out) % 16 == 0,
@@ -268,7 +271,7 @@ extern "C" int mllm_rope_table(const int64_t* positions, int64_t n, const float*
   if (n == 0) return MLLM_OK;
   MLLM_REQUIRE(positions && inv_freq && cos && sin, MLLM_ERR_INVALID, "mllm_rope_table: null pointer");
   const int64_t groups = (n * half + 255) / 256;
-  MLLM_REQUIRE(groups < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_rope_table: too many positions");
+  MLLM_REQUIRE(groups <= kMaxGroups256, MLLM_ERR_UNSUPPORTED, "mllm_rope_table: too many positions");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (dtype == MLLM_DTYPE_BF16)
     rope_table_kernel<BF16><<<(unsigned)groups, 256, 0, st>>>(positions, n, inv_freq, half, (uint16_t*)cos, (uint16_t*)sin);

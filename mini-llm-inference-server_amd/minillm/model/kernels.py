@@ -55,10 +55,13 @@ def _plain_weight(w, like: torch.Tensor) -> bool:
     return type(w) in (torch.nn.Parameter, torch.Tensor) and _rows_ok(w, like)
 
 
+MAX_GROUPS = (1 << 24) - 1  # workgroups of 256 threads one launch takes
+
+
 def norm_ok(x: torch.Tensor, weight) -> bool:
     """Whether `rms_norm` takes x [..., D] (already `usable`) and its weight."""
     d = x.shape[-1]
-    return d % 8 == 0 and x.numel() > 0 and weight.shape == (d,) and _rows_ok(x, x) and _plain_weight(weight, x)
+    return d % 8 == 0 and 0 < x.numel() <= MAX_GROUPS * d and weight.shape == (d,) and _rows_ok(x, x) and _plain_weight(weight, x)
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -78,6 +81,11 @@ def add_rms_norm(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: fl
     return total, out
 
 
+def rope_ok(positions: torch.Tensor, dtype: torch.dtype, half: int) -> bool:
+    return (usable(positions, dtype) and positions.dtype == torch.int64 and positions.is_contiguous()
+            and 0 < positions.numel() * half <= MAX_GROUPS * 256)
+
+
 def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype):
     """cos, sin [..., 2 len(inv_freq)] of int64 positions."""
     half = inv_freq.shape[0]
@@ -93,7 +101,8 @@ def sum_ok(x: torch.Tensor, y: torch.Tensor) -> bool:
 
 
 def silu_mul_ok(gate: torch.Tensor, up: torch.Tensor) -> bool:
-    return usable(gate) and sum_ok(gate, up) and _rows_ok(gate, gate) and gate.numel() % 8 == 0
+    return usable(gate) and sum_ok(gate, up) and _rows_ok(gate, gate) and gate.numel() % 8 == 0 \
+        and gate.numel() <= MAX_GROUPS * 2048
 
 
 def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:

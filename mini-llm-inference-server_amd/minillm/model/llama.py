@@ -55,8 +55,7 @@ class RotaryEmbedding(nn.Module):
 
     def forward(self, positions: torch.Tensor, dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
         """positions [B, T] -> cos, sin [B, T, Dh]: float32 angles, the half-size table repeated."""
-        if kernels.usable(positions, dtype) and positions.dtype == torch.int64 and positions.is_contiguous() \
-                and positions.numel():
+        if kernels.rope_ok(positions, dtype, self._inv_freq.shape[0]):
             return kernels.rope_table(positions, self.inv_freq(positions.device), dtype)
         ang = positions[..., None].float() * self.inv_freq(positions.device)
         ang = torch.cat([ang, ang], dim=-1)

@@ -84,3 +84,15 @@ def test_unaligned_rows_and_large_scores(hip):
     _compare(_run(wide[..., 1:], k, v), torch_ref.prefill(q.double(), k.double(), v.double()), torch.float16)
     q, k = q * 30, k * 30  # scores of some thousands: one key takes all the weight, the max moves far
     _compare(_run(q, k, v), torch_ref.prefill(q.double(), k.double(), v.double()), torch.float16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_more_workgroups_than_a_launch_takes(hip, dtype):
+    # 2^24 and more workgroups of 256 threads are past HIP's 2^32 work-items along x: those calls run on dense_kernel.
+    # One query and one key each, so that a row's result is its value.
+    from minillm.attention import get_backend
+
+    b, h = 4096, 4096
+    v = torch.randn(b, 1, 1, 64, generator=torch.Generator().manual_seed(5)).to(DEV, dtype).expand(b, h, 1, 64)
+    q = k = torch.ones(1, 1, 1, 64, device=DEV, dtype=dtype).expand(b, h, 1, 64)
+    assert torch.equal(get_backend("hip").prefill(q, k, v), v)

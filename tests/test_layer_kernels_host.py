@@ -46,3 +46,25 @@ def test_weights_held_as_plain_attributes():
         delattr(other, name)
         setattr(other, name, value)
         assert not kernels.weights_ok(x, 256, other)
+
+
+def test_more_rows_than_a_launch_takes(monkeypatch):
+    # a launch has fewer than 2^32 threads: larger calls keep torch's expressions, and the entry points refuse them
+    # before they launch anything
+    from minillm import _native
+
+    empty = lambda *s: torch.empty(s, dtype=torch.bfloat16, device="meta")  # noqa: E731
+    assert kernels.norm_ok(empty((1 << 24) - 1, 8), empty(8)) and not kernels.norm_ok(empty(1 << 24, 8), empty(8))
+    monkeypatch.setattr(kernels, "usable", lambda x, dtype=None: True)
+    assert kernels.silu_mul_ok(empty((1 << 35) - 2048), empty((1 << 35) - 2048))
+    assert not kernels.silu_mul_ok(empty(1 << 35), empty(1 << 35))
+    pos = torch.empty(1 << 26, dtype=torch.int64, device="meta")
+    assert not kernels.rope_ok(pos, torch.bfloat16, 64) and kernels.rope_ok(pos[:-4], torch.bfloat16, 64)
+    call, p = _native.lib().call, 1 << 20  # 16-byte aligned, never read
+    for name, args in (("mllm_rms_norm", (p, None, p, 1 << 24, 8, 1e-5, 2, None, p, None)),
+                       ("mllm_silu_mul", (p, p, 1 << 35, 2, p, None)),
+                       ("mllm_sum_partials", (p, 1, 1 << 24, 2048, None, 2, p, None)),
+                       ("mllm_sum_partials_norm", (p, 1, p, p, 1 << 24, 8, 1e-5, 2, p, p, None)),
+                       ("mllm_rope_table", (p, 1 << 26, p, 64, 2, p, p, None))):
+        with pytest.raises(ValueError, match="fewer than|too many"):
+            call(name, *args)
