@@ -290,18 +290,6 @@ int mllm_attention_forward(const mllm_layer_step* step, const void* q, int64_t q
                            float v_scale, void* out, void* stream);
 
 /*
- * mllm_attention_forward with the decode rows among the step's first `rows` sequences (rows > 0: their number) run by
- * one workgroup per row and KV head, whose wavefronts share the row's pages and merge on chip: no decode or merge
- * work of the plan is read, and no workspace.  16-bit pools.  For steps of few, not too long rows; the results
- * differ from the plan's bins in the order of the fp32 sums only.
- */
-int mllm_attention_forward_rows(const mllm_layer_step* step, int32_t rows, const void* q, int64_t q_stride_tok,
-                                int64_t q_stride_head, const void* k, int64_t k_stride_tok, int64_t k_stride_head,
-                                const void* v, int64_t v_stride_tok, int64_t v_stride_head, const void* cos,
-                                const void* sin, int64_t cs_stride_tok, void* q_rot, void* k_cache, void* v_cache,
-                                float k_scale, float v_scale, void* out, void* stream);
-
-/*
  * Contiguous causal attention, the backend's `prefill` method (reference
  * src/minillm/attention/torch_ref.py:20-44 and base.py:19-33): q [B, H, Tq, Dh], k/v [B, Hkv, Tk, Dh]
  * with element strides (batch, head, token) and unit stride on Dh; query i sits at position
@@ -358,8 +346,7 @@ int mllm_linear_swiglu(const void* x, int64_t m, int64_t k, const void* gate, co
 
 /*
  * A whole decoder layer of a paged step of at most 64 rows in one host call (reference src/minillm/model/llama.py:117-127):
- *   h = RMSNorm(x); q, k, v = h . w^T; the step's RoPE, append and attention (mllm_attention_forward, or with rows > 0
- *   mllm_attention_forward_rows);
+ *   h = RMSNorm(x); q, k, v = h . w^T; the step's RoPE, append and attention (mllm_attention_forward);
  *   x2 = x + attn . wo^T; out = x2 + SwiGLU(RMSNorm(x2)) . down^T
  * as the launches of the entry points above, in that order on `stream`, with their limits; x and out [N, hidden], weights as
  * torch.nn.Linear holds them.  `scratch`: mllm_decoder_layer_scratch_bytes bytes, 256-byte aligned, not shared with
@@ -367,7 +354,7 @@ int mllm_linear_swiglu(const void* x, int64_t m, int64_t k, const void* gate, co
  */
 int64_t mllm_decoder_layer_scratch_bytes(int64_t rows, int64_t hidden, int64_t ffn, int32_t num_heads,
                                          int32_t num_kv_heads, int32_t head_dim);
-int mllm_decoder_layer(const mllm_layer_step* step, int32_t rows, const void* x, int64_t hidden, const void* norm1, float eps1,
+int mllm_decoder_layer(const mllm_layer_step* step, const void* x, int64_t hidden, const void* norm1, float eps1,
                        const void* wq, const void* wk, const void* wv, const void* wo, const void* norm2, float eps2,
                        const void* gate, const void* up, const void* down, int64_t ffn, const void* cos,
                        const void* sin, int64_t cs_stride_tok, void* k_cache, void* v_cache, float k_scale,

@@ -26,11 +26,6 @@ int check_launch(const char* what);
 // HIP takes fewer than 2^32 work-items along x: workgroups of 256 threads a launch may have.
 constexpr int64_t kMaxGroups256 = (1ll << 24) - 1;
 
-// Decode of the rows with one new token among the step's first `rows` sequences by row workgroups
-// (decode_rows_kernel): q as given, out [N, H, Dh].
-int paged_decode_rows(const mllm_layer_step& s, const void* q, int64_t q_stride_tok, int64_t q_stride_head,
-                      const void* k_cache, const void* v_cache, int32_t rows, void* out, void* stream);
-
 // ---------------------------------------------------------------- types
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));

@@ -385,96 +385,6 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(OCC,
   }
 }
 
-// Small steps (16-bit pools): one workgroup of W wavefronts per (row, KV head).  Wavefront w streams the w-th part of the
-// row's pages as decode_kernel streams a bin, and the W partial (m, l, O) of the G query heads meet in LDS, so there
-// are no partials in memory, no merge launch and no plan.
-// Bound by latency: the launch, and a wavefront's chain of tiles (one loaded ahead; four ahead at two wavefronts per
-// SIMD measured slower, 14.0 against 10.7 us for 4 rows).  Append + decode of a layer, Llama-3.1-8B heads, bf16,
-// against bins and their merge: 4 rows of 37-500 tokens 10.7 against 11.6 us, 8 rows of 100 8.5 against 10.8, 32 of
-// 200 11.6 against 15.3, 64 of 100 11.8 against 16.3, 96 of 200 21.7 against 25.1; longer rows lose, one CU's
-// wavefronts streaming only some 30 GB/s: 8 rows of up to 1,700 tokens 34.5 against 18.4.
-template <typename T, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) void decode_rows_kernel(
-    const DecodeArgs a) {
-  constexpr int kPad = kHeadDim + 4;  // floats per head row: heads 16 bytes apart in the banks
-  __shared__ __attribute__((aligned(16))) float part[W][16][kPad];
-  __shared__ float2 ml[W][16];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kvh = blockIdx.x % a.Hkv, seq = blockIdx.x / a.Hkv;  // each XCD serves one of 8 KV heads
-  typedef const __attribute__((address_space(4))) int32_t MetaInt;  // uniform and constant: scalar loads
-  const int qrow = ((MetaInt*)a.qo_indptr)[seq];
-  if (((MetaInt*)a.qo_indptr)[seq + 1] - qrow != 1) return;  // not a decode row
-  const int kv0 = ((MetaInt*)a.kv_indptr)[seq], len = ((MetaInt*)a.seq_lens)[seq];
-  // pages past the row's last token (a block table may hold pages ahead) are left out
-  const int pages = min(((MetaInt*)a.kv_indptr)[seq + 1] - kv0, (len + a.bs - 1) / a.bs);
-  const int p0 = pages * wave / W, p1 = pages * (wave + 1) / W;
-  const int tpp = a.bs >> 4;
-  const int c = lane & 15;
-  const int g = lane >> 4;
-  const bool qvalid = c < a.G;
-  const int64_t tok_stride = (int64_t)a.Hkv * kHeadDim * 2;
-  const int64_t blk_stride = (int64_t)a.bs * tok_stride;
-  const char* kbase = a.kc + kvh * kHeadDim * 2;
-  const char* vbase = a.vc + kvh * kHeadDim * 2;
-  float m_run = -INFINITY, l_run = 0.f;
-  f32x4 o[8];
-#pragma unroll
-  for (int m = 0; m < 8; ++m) o[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4 qf[4];
-  {
-    const char* qp =
-        reinterpret_cast<const char*>(a.q + (int64_t)qrow * a.q_st + (int64_t)(kvh * a.G + (qvalid ? c : 0)) * a.q_sh);
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const u32x4 v = ld16(qp + 2 * qk_dim0<false>(kk, g));
-      qf[kk] = qvalid ? v : u32x4{0, 0, 0, 0};
-    }
-  }
-  for (int b0 = p0; b0 < p1; b0 += kMaxSplitPages) {  // as many pages as a lane's registers hold ids for
-    const int b1 = min(b0 + kMaxSplitPages, p1);
-    const PageIds ids = load_page_ids(a.kv_indices, make_int4(kv0 + b0, b1 - b0, 0, 0), lane);
-    const int tok0 = b0 * a.bs;
-    const int ntiles = (min(len, b1 * a.bs) - tok0 + 15) >> 4;
-    TileRegs<false> tile, ahead;
-    LoadCursor at;
-    load_tile<false, true>(a, kbase, vbase, tok_stride, blk_stride, ids, at, c, g, tile);
-    at.advance(tpp);
-    for (int t = 0; t + 1 < ntiles; ++t) {
-      load_tile<false, true>(a, kbase, vbase, tok_stride, blk_stride, ids, at, c, g, ahead);
-      at.advance(tpp);
-      consume_tile<T>(tile.k, tile.v, qf, a.scale_log2, tok0 + t * 16, len, g, m_run, l_run, o);
-      tile = ahead;
-    }
-    consume_tile<T>(tile.k, tile.v, qf, a.scale_log2, tok0 + (ntiles - 1) * 16, len, g, m_run, l_run, o);
-  }
-  if (qvalid) {  // lane (c, g) owns dims 32 g + 8 i + m of head c: o[m][i]
-    float* po = &part[wave][c][32 * g];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<f32x4*>(po + 8 * i) = f32x4{o[0][i], o[1][i], o[2][i], o[3][i]};
-      *reinterpret_cast<f32x4*>(po + 8 * i + 4) = f32x4{o[4][i], o[5][i], o[6][i], o[7][i]};
-    }
-    if (g == 0) ml[wave][c] = make_float2(m_run, l_run);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < a.G * (kHeadDim / 2); i += 64 * W) {  // two dims of one head
-    const int head = i / (kHeadDim / 2), d = 2 * (i % (kHeadDim / 2));
-    float m = -INFINITY, l = 0.f, x = 0.f, y = 0.f;
-#pragma unroll
-    for (int w = 0; w < W; ++w) m = fmaxf(m, ml[w][head].x);
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      const float wgt = fast_exp2(ml[w][head].x - m);  // a wavefront without pages: 2^-inf
-      l += wgt * ml[w][head].y;
-      x += wgt * part[w][head][d];
-      y += wgt * part[w][head][d + 1];
-    }
-    uint16_t* op = a.out + (int64_t)qrow * a.o_st + (int64_t)(kvh * a.G + head) * a.o_sh + d;
-    *reinterpret_cast<uint32_t*>(op) = pack2<T>(x / l, y / l);
-  }
-}
-
 // fp8 pools, two adjacent KV heads per wavefront (heads 2j and 2j + 1).  Their 128-byte rows of one
 // token are one 256-byte row of the pool, so the pair is loaded exactly as the 16-bit kernel loads one
 // head: K row c as four 16-byte pieces (bytes 64 p + 16 g .. +15, p = 0..3; pieces 0-1 are head A's,
@@ -793,9 +703,6 @@ constexpr int max_bins(int n_work) { return n_work >= 4 ? (n_work - 1) / 3 : 0; 
 // that many slots: acc[slot][head][Dh], then (m, l)[slot][head].
 constexpr int partial_slots(int n_work) { return n_work >= 1 ? (n_work - 1) / 2 : 0; }
 
-// Row workgroups (decode_rows_kernel): 12 wavefronts, a CU each, while every one gets a CU, else 4, three to a CU.
-constexpr int kRowsOneRound = 256;
-
 template <typename T, bool F8>
 int launch(const DecodeArgs& a, int n_work, int pages_per_split, hipStream_t st) {
   const unsigned bins = (unsigned)max_bins(n_work);
@@ -821,16 +728,6 @@ int launch(const DecodeArgs& a, int n_work, int pages_per_split, hipStream_t st)
   return check_launch(F8 ? "mllm_paged_decode_fp8" : "mllm_paged_decode");
 }
 
-template <typename T>
-int launch_rows(const DecodeArgs& a, int rows, hipStream_t st) {
-  const unsigned grid = (unsigned)rows * (unsigned)a.Hkv;
-  if (rows * a.Hkv <= kRowsOneRound)
-    decode_rows_kernel<T, 12><<<grid, 64 * 12, 0, st>>>(a);
-  else
-    decode_rows_kernel<T, 4><<<grid, 64 * 4, 0, st>>>(a);
-  return check_launch("mllm_paged_decode_rows");
-}
-
 }  // namespace
 }  // namespace mllm
 
@@ -848,8 +745,7 @@ int paged_decode(const void* q, int64_t q_stride_tok, int64_t q_stride_head, con
                                  const int32_t* decode_work, int32_t num_decode_work, const int32_t* merge_work,
                                  int32_t num_merge_work, int32_t pages_per_split, float softmax_scale, int32_t dtype,
                                  void* out, int64_t out_stride_tok, int64_t out_stride_head, void* workspace,
-                                 int64_t workspace_bytes, bool fp8, float k_scale, float v_scale, void* stream,
-                                 int32_t rows = 0) {
+                                 int64_t workspace_bytes, bool fp8, float k_scale, float v_scale, void* stream) {
   using namespace mllm;
   const std::string fn = fp8 ? "mllm_paged_decode_fp8" : "mllm_paged_decode";
   MLLM_REQUIRE(dtype == MLLM_DTYPE_BF16 || dtype == MLLM_DTYPE_F16, MLLM_ERR_UNSUPPORTED,
@@ -863,12 +759,11 @@ int paged_decode(const void* q, int64_t q_stride_tok, int64_t q_stride_head, con
                fn + ": num_heads must be a multiple of num_kv_heads");
   MLLM_REQUIRE(num_heads / num_kv_heads <= 16, MLLM_ERR_UNSUPPORTED,
                fn + ": at most 16 query heads per KV head");
-  MLLM_REQUIRE(rows > 0 || (pages_per_split >= 1 && pages_per_split <= kMaxSplitPages), MLLM_ERR_INVALID,
+  MLLM_REQUIRE(pages_per_split >= 1 && pages_per_split <= kMaxSplitPages, MLLM_ERR_INVALID,
                fn + ": pages_per_split must be in [1, 192]");
   MLLM_REQUIRE(num_decode_work >= 0 && num_merge_work >= 0, MLLM_ERR_INVALID, fn + ": negative count");
-  if (num_decode_work == 0 && rows == 0) return MLLM_OK;
-  MLLM_REQUIRE(q && k_cache && v_cache && out && qo_indptr && kv_indptr && kv_indices && seq_lens &&
-                   (decode_work || rows > 0),
+  if (num_decode_work == 0) return MLLM_OK;
+  MLLM_REQUIRE(q && k_cache && v_cache && out && qo_indptr && kv_indptr && kv_indices && seq_lens && decode_work,
                MLLM_ERR_INVALID, fn + ": null pointer");
   const int64_t need = num_merge_work ? mllm_decode_workspace_bytes(num_decode_work, num_heads, head_dim) : 0;
   MLLM_REQUIRE(workspace_bytes >= need && (need == 0 || workspace), MLLM_ERR_INVALID,
@@ -906,7 +801,6 @@ int paged_decode(const void* q, int64_t q_stride_tok, int64_t q_stride_head, con
                                         (int64_t)partial_slots(num_decode_work) * num_heads * head_dim * 4);
   (void)merge_work;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (rows > 0) return dtype == MLLM_DTYPE_BF16 ? launch_rows<BF16>(a, rows, st) : launch_rows<F16>(a, rows, st);
   if (dtype == MLLM_DTYPE_BF16)
     return fp8 ? launch<BF16, true>(a, num_decode_work, pages_per_split, st)
                : launch<BF16, false>(a, num_decode_work, pages_per_split, st);
@@ -943,20 +837,6 @@ extern "C" int mllm_paged_decode_fp8(const void* q, int64_t q_stride_tok, int64_
                       merge_work, num_merge_work, pages_per_split, softmax_scale, dtype, out, out_stride_tok,
                       out_stride_head, workspace, workspace_bytes, true, k_scale, v_scale, stream);
 }
-
-namespace mllm {
-
-int paged_decode_rows(const mllm_layer_step& s, const void* q, int64_t q_stride_tok, int64_t q_stride_head,
-                      const void* k_cache, const void* v_cache, int32_t rows, void* out, void* stream) {
-  MLLM_REQUIRE(!s.kv_fp8, MLLM_ERR_UNSUPPORTED, "mllm_paged_decode_rows: 16-bit pools only");
-  MLLM_REQUIRE((int64_t)rows * s.num_kv_heads < (1ll << 31), MLLM_ERR_UNSUPPORTED, "mllm_paged_decode_rows: too many rows");
-  return paged_decode(q, q_stride_tok, q_stride_head, k_cache, v_cache, s.num_blocks, s.block_size, s.num_heads,
-                      s.num_kv_heads, s.head_dim, s.qo_indptr, s.kv_indptr, s.kv_indices, s.seq_lens, nullptr, 0, nullptr,
-                      0, 0, s.softmax_scale, s.dtype, out, (int64_t)s.num_heads * s.head_dim, s.head_dim, nullptr, 0,
-                      false, 1.f, 1.f, stream, rows);
-}
-
-}  // namespace mllm
 
 namespace {
 

@@ -4,14 +4,12 @@
 // entry points; what changes is the host's cost per layer, one foreign call instead of three or four.
 #include "common.h"
 
-namespace {
-
-// mllm_attention_forward_rows; rows = 0: the plan's decode work.
-int attention_forward(const mllm_layer_step* s, int32_t rows, const void* q, int64_t q_stride_tok,
-                      int64_t q_stride_head, const void* k, int64_t k_stride_tok, int64_t k_stride_head, const void* v,
-                      int64_t v_stride_tok, int64_t v_stride_head, const void* cos, const void* sin,
-                      int64_t cs_stride_tok, void* q_rot, void* k_cache, void* v_cache, float k_scale, float v_scale,
-                      void* out, void* stream) {
+extern "C" int mllm_attention_forward(const mllm_layer_step* s, const void* q, int64_t q_stride_tok,
+                                      int64_t q_stride_head, const void* k, int64_t k_stride_tok,
+                                      int64_t k_stride_head, const void* v, int64_t v_stride_tok,
+                                      int64_t v_stride_head, const void* cos, const void* sin, int64_t cs_stride_tok,
+                                      void* q_rot, void* k_cache, void* v_cache, float k_scale, float v_scale,
+                                      void* out, void* stream) {
   using namespace mllm;
   MLLM_REQUIRE(s, MLLM_ERR_INVALID, "mllm_attention_forward: null step");
   MLLM_REQUIRE(s->kv_fp8 || (k_scale == 1.f && v_scale == 1.f), MLLM_ERR_INVALID,
@@ -45,10 +43,7 @@ int attention_forward(const mllm_layer_step* s, int32_t rows, const void* q, int
                               stream);
   }
   if (rc != MLLM_OK) return rc;
-  if (rows > 0) {
-    rc = paged_decode_rows(*s, qa, qa_st, qa_sh, k_cache, v_cache, rows, out, stream);
-    if (rc != MLLM_OK) return rc;
-  } else if (s->num_decode_work > 0) {
+  if (s->num_decode_work > 0) {
     rc = fp8 ? mllm_paged_decode_fp8(qa, qa_st, qa_sh, k_cache, v_cache, s->num_blocks, s->block_size, s->num_heads,
                                      s->num_kv_heads, s->head_dim, s->qo_indptr, s->kv_indptr, s->kv_indices,
                                      s->seq_lens, s->decode_work, s->num_decode_work, s->merge_work,
@@ -76,29 +71,6 @@ int attention_forward(const mllm_layer_step* s, int32_t rows, const void* q, int
                                   s->softmax_scale, s->dtype, out, row, s->head_dim, stream);
   }
   return rc;
-}
-
-}  // namespace
-
-extern "C" int mllm_attention_forward(const mllm_layer_step* s, const void* q, int64_t q_stride_tok,
-                                      int64_t q_stride_head, const void* k, int64_t k_stride_tok,
-                                      int64_t k_stride_head, const void* v, int64_t v_stride_tok,
-                                      int64_t v_stride_head, const void* cos, const void* sin, int64_t cs_stride_tok,
-                                      void* q_rot, void* k_cache, void* v_cache, float k_scale, float v_scale,
-                                      void* out, void* stream) {
-  return attention_forward(s, 0, q, q_stride_tok, q_stride_head, k, k_stride_tok, k_stride_head, v, v_stride_tok,
-                           v_stride_head, cos, sin, cs_stride_tok, q_rot, k_cache, v_cache, k_scale, v_scale, out, stream);
-}
-
-extern "C" int mllm_attention_forward_rows(const mllm_layer_step* s, int32_t rows, const void* q, int64_t q_stride_tok,
-                                      int64_t q_stride_head, const void* k, int64_t k_stride_tok,
-                                      int64_t k_stride_head, const void* v, int64_t v_stride_tok,
-                                      int64_t v_stride_head, const void* cos, const void* sin, int64_t cs_stride_tok,
-                                      void* q_rot, void* k_cache, void* v_cache, float k_scale, float v_scale,
-                                      void* out, void* stream) {
-  MLLM_REQUIRE(rows > 0, MLLM_ERR_INVALID, "mllm_attention_forward_rows: rows must be positive");
-  return attention_forward(s, rows, q, q_stride_tok, q_stride_head, k, k_stride_tok, k_stride_head, v, v_stride_tok,
-                           v_stride_head, cos, sin, cs_stride_tok, q_rot, k_cache, v_cache, k_scale, v_scale, out, stream);
 }
 
 // ---------------------------------------------------------------- a whole decoder layer of few rows
@@ -151,7 +123,7 @@ extern "C" int64_t mllm_decoder_layer_scratch_bytes(int64_t rows, int64_t hidden
   return layer_scratch(rows, hidden, ffn, (int64_t)num_heads * head_dim, (int64_t)num_kv_heads * head_dim).total;
 }
 
-extern "C" int mllm_decoder_layer(const mllm_layer_step* s, int32_t rows, const void* x, int64_t hidden, const void* norm1,
+extern "C" int mllm_decoder_layer(const mllm_layer_step* s, const void* x, int64_t hidden, const void* norm1,
                                   float eps1, const void* wq, const void* wk, const void* wv, const void* wo,
                                   const void* norm2, float eps2, const void* gate, const void* up, const void* down,
                                   int64_t ffn, const void* cos, const void* sin, int64_t cs_stride_tok, void* k_cache,
@@ -176,7 +148,7 @@ extern "C" int mllm_decoder_layer(const mllm_layer_step* s, int32_t rows, const 
   if (rc == MLLM_OK) rc = mllm_linear_partial(h, m, hidden, wq, nq, wk, nkv, wv, nkv, at.ks_qkv, part, dt, stream);
   if (rc == MLLM_OK) rc = mllm_sum_partials(part, at.ks_qkv, m, cols, nullptr, dt, qkv, stream);
   if (rc == MLLM_OK)
-    rc = attention_forward(s, rows, qkv, cols, dh, qkv + 2 * nq, cols, dh, qkv + 2 * (nq + nkv), cols, dh, cos, sin,
+    rc = mllm_attention_forward(s, qkv, cols, dh, qkv + 2 * nq, cols, dh, qkv + 2 * (nq + nkv), cols, dh, cos, sin,
                                 cs_stride_tok, base + at.q_rot, k_cache, v_cache, k_scale, v_scale, attn, stream);
   if (rc == MLLM_OK) rc = mllm_linear_partial(attn, m, nq, wo, hidden, nullptr, 0, nullptr, 0, at.ks_o, part, dt, stream);
   if (rc == MLLM_OK) rc = mllm_sum_partials_norm(part, at.ks_o, x, norm2, m, hidden, eps2, dt, x2, h, stream);

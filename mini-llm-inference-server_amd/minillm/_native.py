@@ -59,8 +59,6 @@ SIGNATURES = {
     # one layer: append (RoPE optionally fused), decode + merge, prefill
     "mllm_attention_forward": (ctypes.c_int, [_p, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _p, _i64, _p,
                                               _p, _p, _f32, _f32, _p, _p]),
-    "mllm_attention_forward_rows": (ctypes.c_int, [_p, _i32, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _p, _i64, _p,
-                                              _p, _p, _f32, _f32, _p, _p]),
     "mllm_paged_prefill": (ctypes.c_int, [_p, _i64, _i64, _p, _p, _i64, _i32, _i32, _i32, _i32, _p, _p, _p, _p, _p,
                                           _i32, _i32, _f32, _i32, _p, _i64, _i64, _p]),
     "mllm_dense_attention": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64,
@@ -75,7 +73,7 @@ SIGNATURES = {
     "mllm_rope_table": (ctypes.c_int, [_p, _i64, _p, _i32, _i32, _p, _p, _p]),
     "mllm_linear_ksplit": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
     "mllm_decoder_layer_scratch_bytes": (ctypes.c_int64, [_i64, _i64, _i64, _i32, _i32, _i32]),
-    "mllm_decoder_layer": (ctypes.c_int, [_p, _i32, _p, _i64, _p, _f32, _p, _p, _p, _p, _p, _f32, _p, _p, _p, _i64, _p, _p, _i64,
+    "mllm_decoder_layer": (ctypes.c_int, [_p, _p, _i64, _p, _f32, _p, _p, _p, _p, _p, _f32, _p, _p, _p, _i64, _p, _p, _i64,
                                           _p, _p, _f32, _f32, _p, _i64, _p, _p]),
     # fp8 (e4m3fn) pools with per-tensor k_scale / v_scale
     "mllm_kv_append_fp8": (ctypes.c_int, [_p, _i64, _i64, _p, _i64, _i64, _i32, _p, _p, _i64, _i32, _i32, _p, _i64, _f32,

@@ -162,30 +162,6 @@ def prefill_q_tile(num_new: list[int], group: int, num_kv_heads: int, kv_fp8: bo
     return (PREFILL_ROWS_SMALL if small else PREFILL_ROWS) // group
 
 
-ROW_GROUPS = 768  # row workgroups resident at once: three of 4 wavefronts on each of 256 CUs
-ROW_TOKENS_ALONE = 512  # longest decode row while each workgroup has a CU to itself (12 wavefronts)
-ROW_TOKENS = 320  # and with 4 wavefronts per workgroup
-
-
-def row_workgroups(num_new: list[int], seq_lens: list[int], num_heads: int, num_kv_heads: int, head_dim: int,
-                   kv_fp8: bool = False) -> int:
-    """The step's sequences if its decode rows run as row workgroups (one per row and KV head, no merge launch), else 0:
-    few enough to be resident at once, and rows short enough that a workgroup's wavefronts get through theirs before
-    bins spread over the whole chip would.  Measured on MI355X (append + decode per layer, Llama-3.1-8B heads, bf16;
-    row workgroups against bins + merge): up to 300 tokens faster at every row count, 100 tokens: 4 rows 8.3 against
-    10.3 us, 32 rows 9.4 against 12.5, 64 rows 11.8 against 16.3; 300 tokens: 11.4 / 12.0, 13.6 / 17.6, 20.5 / 24.2.  At
-    500 tokens 32 rows 18.4 against 20.9 us, 8 rows 15.4 against 13.5 with one launch less for the host (4 rows of
-    37-500 tokens, called eagerly: 19.9 against 22.1 us); 48 rows 27.9 against 26.8.  8 rows of 200-1,000 tokens:
-    21.8 against 15.3 us.  16-bit pools (the fp8 kernels keep bins); a forced bin size keeps bins."""
-    groups = len(seq_lens) * num_kv_heads
-    if groups > ROW_GROUPS or kv_fp8 or head_dim != 128 or os.environ.get("MLLM_PAGES_PER_SPLIT"):
-        return 0
-    longest = max((n for n, new in zip(seq_lens, num_new) if new == 1), default=0)
-    if not longest or longest > (ROW_TOKENS_ALONE if groups <= FULL_CHIP_CUS else ROW_TOKENS):
-        return 0
-    return len(seq_lens)
-
-
 class PlanOverflowError(RuntimeError):
     """A decode plan did not fit the capacities it was given (its header reads {0, records, merges, -1})."""
 
@@ -214,7 +190,6 @@ class StepPlan:
     merge_work: torch.Tensor
     prefill_work: torch.Tensor
     workspace_bytes: int
-    rows: int = 0  # sequences whose decode rows run as row workgroups (row_workgroups), 0: the plan's bins
     # the step's fixed pointer arguments, taken once per plan instead of once per layer: the metadata's
     # qo_indptr, kv_indptr, kv_indices, seq_lens_i32, then the work lists and their sizes
     meta_ptrs: tuple = ()
@@ -270,7 +245,6 @@ class HipBackend(AttentionBackend):
     def __init__(self) -> None:
         self._lib = _native.lib()
         self._attention_forward = self._lib.fn("mllm_attention_forward")
-        self._attention_forward_rows = self._lib.fn("mllm_attention_forward_rows")
         self._planned = None  # the AttentionMetadata the plan was last built for
         self._planned_fp8 = False  # and the pool type it was built for
         self._plan: StepPlan | None = None
@@ -307,20 +281,18 @@ class HipBackend(AttentionBackend):
         plan = self.plan(meta, q.shape[1], k_cache.shape[2], q.shape[2], q.device, fp8)
         step = self._layer_step(plan, meta, q.shape[0], q.shape[1], q.dtype, k_cache, fp8)
         rot = cos is not None
-        head, call = ((step,), self._attention_forward) if not plan.rows else \
-            ((step, plan.rows), self._attention_forward_rows)
-        self._lib.check(call(
-            *head, q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
+        self._lib.check(self._attention_forward(
+            step, q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
             v.stride(0), v.stride(1), cos.data_ptr() if rot else None, sin.data_ptr() if rot else None,
             cos.stride(0) if rot else 0, q_rot.data_ptr() if rot else None, k_cache.data_ptr(), v_cache.data_ptr(),
             k_scale, v_scale, out.data_ptr(), _native.stream_ptr(q.device)))
 
-    def layer_step(self, meta, n: int, num_heads: int, dtype, k_cache) -> tuple[int, int]:
-        """Address of the step's mllm_layer_step for rows of `num_heads` query heads in `dtype` and these pools, and the
-        sequences its decode rows run as row workgroups over (the plan is built on the first call with `meta`)."""
+    def layer_step(self, meta, n: int, num_heads: int, dtype, k_cache) -> int:
+        """Address of the step's mllm_layer_step for rows of `num_heads` query heads in `dtype` and these pools (the
+        plan is built on the first call with `meta`)."""
         fp8 = is_fp8(k_cache)
         plan = self.plan(meta, num_heads, k_cache.shape[2], k_cache.shape[3], k_cache.device, fp8)
-        return self._layer_step(plan, meta, n, num_heads, dtype, k_cache, fp8), plan.rows
+        return self._layer_step(plan, meta, n, num_heads, dtype, k_cache, fp8)
 
     def _layer_step(self, plan: StepPlan, meta, n: int, num_heads: int, dtype, k_cache, fp8: bool) -> int:
         """Address of the plan's mllm_layer_step for these pools and this workspace."""
@@ -535,8 +507,7 @@ class HipBackend(AttentionBackend):
         ws = self._lib.workspace_bytes(n_dec, h, dh) if n_merge else 0
         meta_ptrs = (meta.qo_indptr.data_ptr(), meta.kv_indptr.data_ptr(), meta.kv_indices.data_ptr(),
                      meta.seq_lens_i32.data_ptr())
-        self._plan = StepPlan(c, q_tile, n_dec, n_merge, n_pf, dec, mrg, pf, ws,
-                              0 if split_dev is not None else row_workgroups(news, lens, h, hkv, dh, kv_fp8), meta_ptrs,
+        self._plan = StepPlan(c, q_tile, n_dec, n_merge, n_pf, dec, mrg, pf, ws, meta_ptrs,
                               (*meta_ptrs, _ptr(dec), n_dec, _ptr(mrg), n_merge, c))
         self._planned, self._planned_fp8 = meta, kv_fp8
         if self.check_plan and n_dec and not torch.cuda.is_current_stream_capturing():

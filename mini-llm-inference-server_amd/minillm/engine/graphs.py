@@ -122,7 +122,7 @@ class DecodeGraphs:
 
     def _split(self, pages: int) -> int:
         """The split size an eager step over `pages` decode pages uses with this pool.  A replay cuts the same
-        bins (steps that eagerly run as row workgroups differ in the order of their fp32 sums); its decode launch, planned at the smallest
+        bins, so its output is the eager step's bit for bit; its decode launch, planned at the smallest
         split, runs 4-wavefront workgroups over them (the launch shape does not change a wavefront's
         arithmetic)."""
         return pages_per_split(pages, self.num_kv_heads, self.num_heads, self.cache.quantized,

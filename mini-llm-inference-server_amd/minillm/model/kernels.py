@@ -226,9 +226,9 @@ def decoder_layer(layer, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, 
     ffn = gate.shape[0]
     scratch = torch.empty(lib.fn("mllm_decoder_layer_scratch_bytes")(n, d, ffn, h, hkv, dh), dtype=torch.uint8,
                           device=x.device)
-    step, rows = backend.layer_step(meta, n, h, x.dtype, kc)
+    step = backend.layer_step(meta, n, h, x.dtype, kc)
     out = torch.empty_like(x)
-    lib.call("mllm_decoder_layer", step, rows, x.data_ptr(), d, norm1.weight.data_ptr(), norm1.eps, wq.data_ptr(), wk.data_ptr(),
+    lib.call("mllm_decoder_layer", step, x.data_ptr(), d, norm1.weight.data_ptr(), norm1.eps, wq.data_ptr(), wk.data_ptr(),
              wv.data_ptr(), attn.o_proj.weight.data_ptr(), norm2.weight.data_ptr(), norm2.eps, gate.data_ptr(),
              mlp.up_proj.weight.data_ptr(), mlp.down_proj.weight.data_ptr(), ffn, cos.data_ptr(), sin.data_ptr(),
              dh, kc.data_ptr(), vc.data_ptr(), ks, vs, scratch.data_ptr(), scratch.numel(), out.data_ptr(),

@@ -61,6 +61,45 @@ def test_graph_engine_matches_eager_engine(hip, kv):
     assert core.graphs.replays > 10 and len(core.graphs._captured) >= 2  # batch shrinks as requests finish
 
 
+@pytest.mark.parametrize("steps", [
+    [(37, 1), (128, 1), (211, 1), (500, 1)], [(17 * i % 300, 1) for i in range(40)], [(90, 1), (0, 30), (250, 1), (7, 5)]],
+    ids=["4_rows", "40_rows", "mixed"])
+def test_a_step_is_the_same_bits_by_every_route(hip, steps):
+    # one call per layer, separate launches, prefill on a second stream, and (decode steps) the staged metadata of a
+    # captured graph whose bucket the step fills: short rows too are cut into the same bins
+    from minillm.attention.hip_backend import HipBackend, device_cus, pages_per_split
+    from minillm.attention.metadata import AttentionMetadata, DeviceBlockTables, SeqStep, StaticDecodeMetadata
+    from test_gpu_paged import _kernel_case, bits
+
+    blocks = sum(-(-(c + n) // 16) for c, n in steps)
+    wl = _kernel_case(32, 8, 128, 16, torch.bfloat16, steps, seed=71, num_blocks=blocks + 4)
+    q, k, v = wl.q.to(DEV), wl.k.to(DEV), wl.v.to(DEV)
+    seqs = [SeqStep(c, n, list(b)) for c, n, b in wl.seqs]
+    results = {}
+    for route in ("one_call", "separate", "second_stream", "staged"):
+        be, pk, pv = HipBackend(), wl.pool_k.to(DEV), wl.pool_v.to(DEV)
+        if route == "staged":
+            if any(n > 1 for _, n in steps):
+                continue
+            static = StaticDecodeMetadata(len(seqs), DeviceBlockTables(len(seqs), blocks, DEV), 16)
+            static.load(list(range(len(seqs))), seqs, pages_per_split(blocks, 8, 32, False, device_cus(DEV)))
+            static.build()
+            meta = static.meta
+        else:
+            meta = AttentionMetadata.build(seqs, 16, DEV)
+        if route == "separate":
+            out = torch.empty_like(q)
+            be.append(k, v, pk, pv, meta)
+            be.attend(q, pk, pv, meta, out)
+        else:
+            be.overlap_mixed = route == "second_stream"
+            out = be.forward(q, k, v, pk, pv, meta)
+        torch.cuda.synchronize()
+        results[route] = out
+    for route, out in results.items():
+        assert torch.equal(bits(out), bits(results["one_call"])), route
+
+
 def test_host_running_ahead_of_the_gpu_changes_nothing(hip):
     # a sampler that returns its tokens without reading the GPU lets the host stage the next replay while
     # the GPU still works on earlier steps (held back here by a bounded spin kernel per step): the staged

@@ -287,43 +287,3 @@ def test_decoder_layer_in_one_call(hip, dtype, kv, rows):
             results.append((layer(x, cos, sin, step), cache.k[0], cache.v[0]))
     for a, b in zip(*results):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("h,hkv,bs,steps", [
-    (8, 2, 16, [(0, 1), (14, 1), (15, 1), (16, 1), (191, 1), (511, 1)]),  # 12 wavefronts: none, one and several tiles each
-    (4, 4, 32, [(300, 1), (0, 9), (31, 1), (100, 3)]),  # one head per KV head, other block size, rows of several tokens
-    (16, 1, 16, [(250, 1)] * 3),  # 16 heads per KV head
-    (32, 8, 16, [(17 * i % 300, 1) for i in range(33)]),  # 264 workgroups: 4 wavefronts each
-    (2, 1, 16, [(40000, 1), (5, 1)])])  # more than 192 pages per wavefront (the rule would not pick it)
-def test_row_workgroups(hip, monkeypatch, dtype, h, hkv, bs, steps):
-    from minillm.attention import hip_backend
-    from test_gpu_paged import ATOL, RTOL, _kernel_case, bits, hip_step, oracle_step
-
-    monkeypatch.delenv("MLLM_PAGES_PER_SPLIT", raising=False)
-    blocks = sum(-(-(c + n) // bs) for c, n in steps) + 4
-    wl = _kernel_case(h, hkv, 128, bs, dtype, steps, seed=23, num_blocks=blocks)
-    if max(c for c, _ in steps) > 1000:
-        monkeypatch.setattr(hip_backend, "ROW_TOKENS_ALONE", 1 << 20)
-    be = hip_backend.HipBackend()
-    out, pk, pv, meta = hip_step(wl, DEV, backend=be)
-    assert be._plan.rows == len(steps)
-    ref, rk, rv = oracle_step(wl, DEV)
-    assert torch.equal(bits(pk), bits(rk)) and torch.equal(bits(pv), bits(rv))
-    torch.testing.assert_close(out.float(), ref.float(), atol=ATOL, rtol=RTOL)
-    # against the bins and their merge over the same pools: a 16-bit weight is rounded below another running max, so it
-    # may differ by two roundings, 2 EPS of itself; the weights sum to 1 and |v| averages 0.8: 2 EPS in all
-    bins = torch.empty_like(out)
-    be.attend(wl.q.to(DEV), pk, pv, meta, bins)
-    torch.testing.assert_close(out.float(), bins.float(), rtol=2.02 * EPS[dtype], atol=2 * EPS[dtype])
-
-
-def test_row_workgroup_rule():
-    from minillm.attention.hip_backend import row_workgroups
-
-    assert row_workgroups([1] * 4, [38, 129, 212, 501], 32, 8, 128) == 4
-    assert row_workgroups([1] * 4, [38, 129, 212, 513], 32, 8, 128) == 0
-    assert row_workgroups([1] * 33, [320] * 33, 32, 8, 128) == 33 and row_workgroups([1] * 33, [321] * 33, 32, 8, 128) == 0
-    assert row_workgroups([1] * 97, [10] * 97, 32, 8, 128) == 0
-    assert row_workgroups([5, 1], [9000, 30], 8, 2, 128) == 2 and row_workgroups([5, 7], [9, 7], 8, 2, 128) == 0
-    assert row_workgroups([1], [10], 32, 8, 128, kv_fp8=True) == 0
