@@ -12,8 +12,8 @@
 //   dense_kernel        everything else (any Dh up to 256, any strides), one workgroup per query row, fp32 scalar
 //                       arithmetic.
 // Scores and the running max and sum are fp32 everywhere.  The 16-bit MFMA kernels give the PV product the fp32
-// probabilities as two 16-bit operands, P = hi + lo (lo = the rounding error of hi), so that a weight keeps
-// 16 significant bits or more instead of the 8 of a bf16 P.
+// probabilities as a sum of 16-bit operands, each the rounding error of those before it: three in bf16 (8 bits each:
+// the fp32 value), two in fp16 (22 bits: the fp32 value to one unit of its last place).
 #include <math.h>
 
 #include "common.h"
@@ -147,17 +147,18 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(const DenseArgs a) {
 // Per wavefront: 32 query rows (row = token * G + head of the G query heads that share the KV head), keys in
 // tiles of 32 NB:
 //   S^T[keys x 32 rows] = K . Q^T     v_mfma_f32_32x32x16 (K rows by ds_read_b128; Q^T in VGPRs)
-//   O^T[Dh x 32 rows]  += V^T . P^T   v_mfma_f32_32x32x16, once with P's high and once with its low part
+//   O^T[Dh x 32 rows]  += V^T . P^T   v_mfma_f32_32x32x16, once with each part of P
 //                                     (V^T by ds_read_b64_tr_b16, the LDS transpose read)
 // S^T and P^T share a lane layout (lane l: row l % 32), so P never leaves its lanes.  Tiles reach LDS by direct
 // global->LDS loads, one 2 Dh-byte key row after the other, the 16-byte chunks of row r XOR-swizzled so that
 // the operand reads hit distinct banks: Dh 128: K chunk ^ (r % 16), V chunk ^ 4 (r % 4); Dh 64 (two rows per
 // 256 bytes of banks): K chunk ^ (r / 2 % 8), V chunk ^ 4 (r / 2 % 2).  Keys past a workgroup's last visible key
 // are loaded as copies of that key's row and masked.
-// Bound by the MFMA streams (three products' worth per tile with the split P) and, for few rows, by a tile's
-// latency chain.  Against one workgroup per row on the vector ALU, bf16, 32 query and 8 KV heads, Dh 128: one
-// sequence of 512 tokens 637.6 -> 11.4 us a call, four left-padded of 777 3,776 -> 43.9 us, the same distance from
-// float64 (1.6e-3 and 4.8e-4 relative: the output's rounding).
+// Bound by the MFMA streams (with P in three parts four products' worth per tile, in two three) and, for few rows, by a
+// tile's latency chain.  Against one workgroup per row on the vector ALU, bf16, 32 query and 8 KV heads, Dh 128: one
+// sequence of 512 tokens 637.6 -> 11.5 us a call, four left-padded of 777 3,776 -> 49.0 us, the same distance from
+// float64 (1.6e-3 and 4.8e-4 relative: the output's rounding).  P as two bf16 parts took 11.3 and 44.1 us, but left the
+// weights 16 bits: sums that cancel were off by 6e-7 of the values where fp32 weights leave 1e-7.
 // A masked key has P = 0, and 0 x V is 0 only while V is finite: rows whose result is NaN are computed again
 // key by key (row_by_key), which skips the keys of zero weight.
 
@@ -304,20 +305,26 @@ __device__ __forceinline__ void row_by_key(const DenseArgs& a, int b, int h, int
     if (64 * e + lane < a.Dh) st_elem<DT>(a.out, o + 64 * e + lane, acc[e] / l_run);
 }
 
+// The float value of the low / high half of a packed pair; P's 16-bit parts, the power of 2 it is kept larger by, and by
+// how many powers a row's max may grow before its sums are rescaled.
 template <typename T>
-struct Half;  // the float value of the low / high half of a packed pair; the exponent bias of P
+struct Half;
 template <>
 struct Half<BF16> {
   static constexpr int kDt = MLLM_DTYPE_BF16;
-  static constexpr float kBias = 0.f;
+  static constexpr int kParts = 3;
+  static constexpr float kBias = 0.f, kSlack = 8.f;
   static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
   static __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 };
 template <>
 struct Half<F16> {
   static constexpr int kDt = MLLM_DTYPE_F16;
-  // P is kept 2^6 larger (at most 2^14 with the lazy rescale): its low parts stay clear of fp16's subnormals
-  static constexpr float kBias = 6.f;
+  static constexpr int kParts = 2;
+  // The parts end at fp16's smallest step, 2^-24, so P fills the range up to 65,504 (at most 2^15.9): the step is then
+  // 2^-39 of the row's largest weight or less, and a weight 2^-24 of it still has 15 bits.  2^6 larger with a slack of
+  // 8 left that weight 6 bits.
+  static constexpr float kBias = 15.f, kSlack = 0.9f;
   static __device__ __forceinline__ float lo(uint32_t w) { return f16_bits_to_f32((uint16_t)w); }
   static __device__ __forceinline__ float hi(uint32_t w) { return f16_bits_to_f32((uint16_t)(w >> 16)); }
 };
@@ -346,11 +353,11 @@ __device__ __forceinline__ void score_tile(const char* lds, unsigned kb, const u
 }
 
 // Online softmax (exp2 domain) of one tile's scores (keys kv0 .. kv0 + 32 NB - 1): masks, moves the running max
-// when some row's grew by more than 2^8, and leaves P's two 16-bit parts in ph / pl.  vm: the tile's real keys
+// when some row's grew by more than 2^kSlack, and leaves P's 16-bit parts in pp.  vm: the tile's real keys
 // (all ones without a mask); rows without a real key (qp < first) keep only their own position.  A row may meet
 // whole masked tiles before its first key (m = -inf): its P and sum then stay 0.
 template <typename T, int DH, int NB, bool MASKED>
-__device__ __forceinline__ void softmax_tile(f32x16 (&s)[NB], u32x4 (&ph)[NB][2], u32x4 (&pl)[NB][2], RowState<DH>& st,
+__device__ __forceinline__ void softmax_tile(f32x16 (&s)[NB], u32x4 (&pp)[Half<T>::kParts][NB][2], RowState<DH>& st,
                                              int kv0, int qp, int wave_qp_lo, int first, uint64_t vm, int h, float c) {
   constexpr uint64_t kAll = NB == 2 ? ~0ull : 0xffffffffull;
   if (MASKED && vm != kAll) {
@@ -383,7 +390,7 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&s)[NB], u32x4 (&ph)[NB][2]
     for (int r = 0; r < 16; ++r)
       if (b > 0 || r >= 4) m4[r & 3] = __builtin_fmaxf(m4[r & 3], s[b][r]);
   const float mx = max_xor32(__builtin_fmaxf(__builtin_fmaxf(m4[0], m4[1]), __builtin_fmaxf(m4[2], m4[3])));
-  if (__any((mx - st.m) * c > 8.f)) {
+  if (__any((mx - st.m) * c > Half<T>::kSlack)) {
     const float m_new = fmaxf(st.m, mx);
     const float alpha = m_new == st.m ? 1.f : fast_exp2((st.m - m_new) * c);  // -inf - -inf is no rescale
     st.l *= alpha;
@@ -402,10 +409,14 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&s)[NB], u32x4 (&ph)[NB][2]
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float p0 = s[b][8 * u + 2 * e], p1 = s[b][8 * u + 2 * e + 1];
-        const uint32_t w = pack2<T>(p0, p1);
-        ph[b][u][e] = w;
-        pl[b][u][e] = pack2<T>(p0 - Half<T>::lo(w), p1 - Half<T>::hi(w));
+        float p0 = s[b][8 * u + 2 * e], p1 = s[b][8 * u + 2 * e + 1];
+#pragma unroll
+        for (int i = 0; i < Half<T>::kParts; ++i) {
+          const uint32_t w = pack2<T>(p0, p1);
+          pp[i][b][u][e] = w;
+          p0 -= Half<T>::lo(w);
+          p1 -= Half<T>::hi(w);
+        }
       }
   float s4[4] = {s[0][0], s[0][1], s[0][2], s[0][3]};
 #pragma unroll
@@ -418,7 +429,7 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&s)[NB], u32x4 (&ph)[NB][2]
 
 // O^T += V^T P^T for one tile at LDS byte `vb` (this lane's v_read offset within it).
 template <typename T, int DH, int NB>
-__device__ __forceinline__ void pv_tile(const char* lds, unsigned vb, const u32x4 (&ph)[NB][2], const u32x4 (&pl)[NB][2],
+__device__ __forceinline__ void pv_tile(const char* lds, unsigned vb, const u32x4 (&pp)[Half<T>::kParts][NB][2],
                                         RowState<DH>& st) {
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -429,8 +440,8 @@ __device__ __forceinline__ void pv_tile(const char* lds, unsigned vb, const u32x
         const char* p = lds + (vb ^ (64u * dt)) + 16 * (2 * b + u) * Geo<DH>::kRow;
         const u32x2 lo = ld_tr(p), hi = ld_tr(p + 8 * Geo<DH>::kRow);
         const u32x4 vt = u32x4{lo[0], lo[1], hi[0], hi[1]};
-        st.o[dt] = Mfma<T>::m32x32x16(vt, ph[b][u], st.o[dt]);
-        st.o[dt] = Mfma<T>::m32x32x16(vt, pl[b][u], st.o[dt]);
+#pragma unroll
+        for (int i = 0; i < Half<T>::kParts; ++i) st.o[dt] = Mfma<T>::m32x32x16(vt, pp[i][b][u], st.o[dt]);
       }
     }
 }
@@ -564,10 +575,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   barrier_vm<0>();
 
   f32x16 s[2];
-  u32x4 ph[2][2], pl[2][2];
+  u32x4 pp[Half<T>::kParts][2][2];
   if (ts * kBN <= wave_qp_hi) {
     score_tile<T, DH, 2>(lds, kread, qf, s);
-    softmax_tile<T, DH, 2, MASKED>(s, ph, pl, st, ts * kBN, qp, wave_qp_lo, km.first, key_word(ts), h, c);
+    softmax_tile<T, DH, 2, MASKED>(s, pp, st, ts * kBN, qp, wave_qp_lo, km.first, key_word(ts), h, c);
   }
   barrier_lds();  // K(ts) has been read
 
@@ -578,11 +589,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const bool do_pv = j * kBN <= wave_qp_hi, do_s = j + 1 < ntiles && (j + 1) * kBN <= wave_qp_hi;
     const unsigned vb = vread + (j - ts) % 2 * kTile, kb = kread + (j + 1 - ts) % 3 * kTile;
     __builtin_amdgcn_s_setprio(1);
-    if (do_pv) pv_tile<T, DH, 2>(lds, vb, ph, pl, st);
+    if (do_pv) pv_tile<T, DH, 2>(lds, vb, pp, st);
     if (do_s) score_tile<T, DH, 2>(lds, kb, qf, s);
     __builtin_amdgcn_s_setprio(0);
     if (do_s)
-      softmax_tile<T, DH, 2, MASKED>(s, ph, pl, st, (j + 1) * kBN, qp, wave_qp_lo, km.first, key_word(j + 1), h, c);
+      softmax_tile<T, DH, 2, MASKED>(s, pp, st, (j + 1) * kBN, qp, wave_qp_lo, km.first, key_word(j + 1), h, c);
     if (k_ahead)
       barrier_vm<kDma>();
     else
@@ -713,17 +724,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (; t < ntiles; t += 4) {
     const bool more = t + 4 < ntiles;
     f32x16 s[1];
-    u32x4 ph[1][2], pl[1][2];
+    u32x4 pp[Half<T>::kParts][1][2];
     wait_vm<kDma>();  // K(t) has landed (V(t) is younger)
     score_tile<T, DH, 1>(lds, kread, qf, s);
     wait_lds();  // K(t) has been read
     if (more) dma(kc, k_stb, koff, t + 4, kbuf);
-    softmax_tile<T, DH, 1, MASKED>(s, ph, pl, st, t * kBN, qp, qp_lo, km.first, key_word(t), h, c);
+    softmax_tile<T, DH, 1, MASKED>(s, pp, st, t * kBN, qp, qp_lo, km.first, key_word(t), h, c);
     if (more)
       wait_vm<kDma>();
     else
       wait_vm<0>();
-    pv_tile<T, DH, 1>(lds, vread, ph, pl, st);
+    pv_tile<T, DH, 1>(lds, vread, pp, st);
     wait_lds();
     if (more) dma(vc, v_stb, voff, t + 4, vbuf);
   }

@@ -3,6 +3,8 @@ edges of the 16-, 32- and 64-key tiles and of the 16-, 32- and 128-row workgroup
 group size, padding masks (whole padded tiles, windows past 4,096 keys, rows without a real key), unaligned
 views, and values that are not finite behind masked keys.  Against the oracle in float64."""
 
+import math
+
 import pytest
 import torch
 
@@ -75,6 +77,54 @@ def test_values_behind_masked_keys_do_not_leak(hip, dtype, h):
         seen = out[0, :, 40:, 7].float()
         assert (torch.isnan(seen) if bad != bad else seen == bad).all()
         _compare(out[0, :, 40:, 8:], ref[0, :, 40:, 8:], dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("b,h", [(1, 4), (3, 128)])  # workgroups of 32 and of 128 query rows
+def test_weights_keep_fp32_precision(hip, dtype, b, h):
+    # values of +-1 whose signs make the last query's weighted sum cancel, so that the error of the weights shows where
+    # the output's rounding is far smaller; queries and keys of few bits and a scale of 1 / 8, so that the scores are exact
+    t, dh = 128, 64
+    q, k, _ = ((4 * x.float()).round().div(4).to(dtype) for x in _inputs(b, h, h, t, t, dh, dtype, seed=6))
+    q = 2 * q
+    p = torch.softmax((q[:, :, -1:].double() @ k.double().transpose(2, 3))[:, :, 0] * dh ** -0.5, -1)
+    order = p.argsort(-1, descending=True)
+    sign = (torch.rand(b, h, t, dh, generator=torch.Generator().manual_seed(7)) < 0.5).double() * 2 - 1
+    total = torch.zeros(b, h, dh, dtype=torch.float64)
+    for j in range(t):  # the eight largest weights at random, then each against the sum so far
+        if j >= 8:
+            sign[:, :, j] = torch.where(total > 0, -1.0, 1.0)
+        total += p.gather(-1, order[..., j:j + 1]) * sign[:, :, j]
+    v = torch.empty(b, h, t, dh).scatter_(2, order[..., None].expand(b, h, t, dh), sign.float()).to(dtype)
+    got = _run(q, k, v)[:, :, -1].double()
+    small = total.abs() < 2.0 ** -16
+    assert int(small.sum()) > 100
+    rms = (got - total)[small].square().mean().sqrt().item()
+    # fp32 weights: off by two units of 2^-23 of themselves in random directions, and the squares of the weights sum to
+    # about 0.3^2: 7e-8.  The sums: some ten additions rounded at 2^-25 of values below 1: 9e-8.  The output: 2^-9 of 2^-16.
+    assert rms < 1.5e-7, rms
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("b,h", [(1, 4), (3, 128)])
+def test_small_weights_keep_their_precision(hip, dtype, b, h):
+    # key 0 takes nearly all the weight and has the value 0: what is left is the weight of key 1, 2^-4 to 2^-24, times a
+    # large value
+    t, dh = 128, 128
+    q, k, v = (torch.zeros(b, h, t, dh) for _ in range(3))
+    q[..., 0] = 16.0
+    k[..., 0] = -48.0
+    k[:, :, 0, 0] = 0.0
+    drop = torch.linspace(4, 24, b * h).view(b, h)  # log2 of the weights' ratio
+    k[:, :, 1, 0] = -drop * math.log(2) * dh ** 0.5 / 16
+    v[:, :, 1] = 60000.0
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    ref = torch_ref.prefill(q.double(), k.double(), v.double())[:, :, -1]
+    got = _run(q, k, v)[:, :, -1].double()
+    # one rounding of the output; the exponent's 2^-24 of up to 17, and for fp16 weights the grid of their low part,
+    # 2^-39 of the largest weight: 2^-15 covers both
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
+    torch.testing.assert_close(got, ref, rtol=1.01 * eps + 2.0 ** -15, atol=0)
 
 
 def test_unaligned_rows_and_large_scores(hip):
