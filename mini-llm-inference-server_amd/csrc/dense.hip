@@ -159,8 +159,9 @@ __global__ __launch_bounds__(kThreads) void dense_kernel(const DenseArgs a) {
 // sequence of 512 tokens 637.6 -> 11.5 us a call, four left-padded of 777 3,776 -> 49.0 us, the same distance from
 // float64 (1.6e-3 and 4.8e-4 relative: the output's rounding).  P as two bf16 parts took 11.3 and 44.1 us, but left the
 // weights 16 bits: sums that cancel were off by 6e-7 of the values where fp32 weights leave 1e-7.
-// A masked key has P = 0, and 0 x V is 0 only while V is finite: rows whose result is NaN are computed again
-// key by key (row_by_key), which skips the keys of zero weight.
+// A masked key has P = 0, and 0 x V is 0 only while V is finite; the sums of values near the largest may overflow where
+// a weight of at most 1 would not (P is larger by up to 2^kSlack).  Rows whose result is not finite are therefore computed
+// again key by key (row_by_key), which skips the keys of zero weight and has no weight above 1.
 
 template <int DH>
 struct Geo {
@@ -459,14 +460,15 @@ __device__ __forceinline__ void load_q(const DenseArgs& a, int b, int head, int 
   }
 }
 
-// Bit n: row n (of the wavefront's 32) has a NaN among this lane pair's values.
+__device__ __forceinline__ bool not_finite(float x) { return !(__builtin_fabsf(x) < INFINITY); }
+// Bit n: row n (of the wavefront's 32) has a value that is not finite among this lane pair's.
 template <int N>
-__device__ __forceinline__ uint32_t nan_rows(const f32x16 (&o)[N]) {
+__device__ __forceinline__ uint32_t bad_rows_of(const f32x16 (&o)[N]) {
   bool bad = false;
 #pragma unroll
   for (int dt = 0; dt < N; ++dt)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) bad |= o[dt][r] != o[dt][r];
+    for (int r = 0; r < 16; ++r) bad |= not_finite(o[dt][r]);
   const uint64_t m = __ballot(bad);
   return (uint32_t)m | (uint32_t)(m >> 32);
 }
@@ -604,7 +606,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float inv = 1.f / st.l;
 #pragma unroll
   for (int dt = 0; dt < G::kDt; ++dt) st.o[dt] *= inv;
-  uint32_t bad = nan_rows<G::kDt>(st.o);
+  uint32_t bad = bad_rows_of<G::kDt>(st.o);
   char* ost = lds + wave * (32 * G::kRow);
 #pragma unroll
   for (int dt = 0; dt < G::kDt; ++dt)
@@ -767,7 +769,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int w = 0; w < 4; ++w) v += wgt[w] * part[w * kPart + (16 * wave + r) * 64 + lane];
       o[0][r] = v * inv;
     }
-    const uint32_t bad = nan_rows<1>(o);
+    const uint32_t bad = bad_rows_of<1>(o);
     if (bad && lane == 0) atomicOr(&bad_rows, bad);
   }
   __syncthreads();
@@ -950,7 +952,7 @@ __global__ __launch_bounds__(64 * kWavesF32) void dense_f32_kernel(const DenseAr
       }
       res[u] = v / l;
       const f32x4 z = res[u];
-      if (z[0] != z[0] || z[1] != z[1] || z[2] != z[2] || z[3] != z[3]) atomicOr(&bad_rows, 1u << row);
+      if (not_finite(z[0]) || not_finite(z[1]) || not_finite(z[2]) || not_finite(z[3])) atomicOr(&bad_rows, 1u << row);
     }
   }
   __syncthreads();

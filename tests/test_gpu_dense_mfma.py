@@ -127,6 +127,21 @@ def test_small_weights_keep_their_precision(hip, dtype, b, h):
     torch.testing.assert_close(got, ref, rtol=1.01 * eps + 2.0 ** -15, atol=0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b,h", [(1, 4), (2, 128)])
+def test_values_near_the_largest_stay_finite(hip, dtype, b, h):
+    # key 200's score lies 2^7.5 above the rest, which holds the running max back, and its value is 2^-3 of the largest
+    # there is: the output, a little less than that value, is finite however the sums are scaled on the way
+    t, dh = 300, 64
+    q, k, v = (torch.zeros(b, h, t, dh) for _ in range(3))
+    q[..., 0] = 8.0
+    k[:, :, 200, 0] = 7.5 * math.log(2)
+    v[:, :, 200] = 4.2e37
+    v[:, :, 200, 1::2] = -4.2e37
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    _compare(_run(q, k, v) * 2.0 ** -120, torch_ref.prefill(q.double(), k.double(), v.double()) * 2.0 ** -120, dtype)
+
+
 def test_unaligned_rows_and_large_scores(hip):
     q, k, v = _inputs(1, 4, 2, 50, 80, 64, torch.float16, seed=4)
     wide = torch.zeros(1, 4, 50, 65, dtype=torch.float16)
