@@ -303,6 +303,10 @@ int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st
                          int32_t num_kv_heads, int32_t q_len, int32_t kv_len, int32_t head_dim, float softmax_scale,
                          int32_t dtype, void* out, int64_t o_sb, int64_t o_sh, int64_t o_st, void* stream);
 
+/* Query rows (tokens x query heads that share a KV head) per workgroup mllm_dense_attention takes for a bf16 or fp16 call
+ * of this shape on its MFMA kernels: 128 or 32 (0: no such call). */
+int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t q_len);
+
 /*
  * RMSNorm of `rows` contiguous rows of `dim` elements (reference src/minillm/model/llama.py:37-49):
  * out = weight * T(x * rsqrt(mean(x^2) + eps)), fp32 arithmetic, T the 16-bit `dtype` (BF16 or F16).  With

@@ -982,31 +982,42 @@ bool mfma_operands(const DenseArgs& a, int per16) {
          a.v_st < (1 << 24) && a.scale > 0.f && a.scale < INFINITY && a.Tk < (1 << 30);
 }
 
-// Workgroups of 128 rows from 1.5 per CU of the full chip (256) on, else of 32.  Measured (bf16, 32 query and 8 KV
-// heads, Dh 128; 128 rows against 32): 128 workgroups of 128 rows (one sequence of 512 tokens) 19.6 against 11.5 us,
-// 256 (one of 1,024) 34.6 against 27.1 us, 400 (two of 777) 32.8 against 35.4 us, 512 (four of 512) 24.8 against
-// 34.6 us, 800 (four of 777) 42.5 against 65.1 us.  A workgroup of 32 rows reads four times the K and V per row.
-constexpr int64_t kLargeMin = 384;
-
 // Workgroups of `rows` query rows.
 int64_t items(const DenseArgs& a, int rows) {
   const int tokens = rows / a.G;
   return (int64_t)((a.Tq + tokens - 1) / tokens) * a.B * (a.H / a.G);
 }
 
+// Rows per workgroup of the 16-bit kernels: 128 from 1.5 workgroups per CU of the full chip (256) on, if they are fewer than those of 32, else 32.
+// Measured (bf16, 32 query and 8 KV heads, Dh 128; 128 rows against 32, us): 128 workgroups of 128 rows (one sequence of
+// 512 tokens) 23.4 / 12.5, 256 (one of 1,024) 41.0 / 29.8, 400 (two of 777) 39.0 / 38.4, 384 (four of 384) 21.7 / 26.3,
+// 512 (four of 512) 28.2 / 38.6, 800 (four of 777) 49.4 / 68.8: a workgroup of 32 rows reads four times the K and V per
+// row.  Where one workgroup of either size holds all of a head's queries, the 128-row one leaves wavefronts without a row,
+// and one that has some walks all the keys: 1 or 8 queries on 1,024 keys, 64 sequences 47.4 / 43.0 and 48.2 / 43.8, 12 queries
+// (two workgroups of 32 rows) 56.2 / 82.9.
+constexpr int64_t kLargeMin = 384;
+int mfma_rows(const DenseArgs& a) {
+  const int64_t large = items(a, 128);
+  return large >= kLargeMin && large < items(a, 32) ? 128 : 32;
+}
+
+// Query heads of one KV head that share a row of the 16-bit kernels' workgroups.
+int mfma_pack(int group) { return 32 % group == 0 ? group : 1; }
+
 template <typename T, int DH>
 int launch_mfma(const DenseArgs& a, hipStream_t st) {
-  const int64_t large = items(a, 128), small = items(a, 32);
-  if (large >= kLargeMin) {
+  const int rows = mfma_rows(a);
+  const unsigned groups = (unsigned)items(a, rows);
+  if (rows == 128) {
     if (a.key_valid)
-      dense_mfma_kernel<T, DH, true><<<(unsigned)large, 256, 0, st>>>(a);
+      dense_mfma_kernel<T, DH, true><<<groups, 256, 0, st>>>(a);
     else
-      dense_mfma_kernel<T, DH, false><<<(unsigned)large, 256, 0, st>>>(a);
+      dense_mfma_kernel<T, DH, false><<<groups, 256, 0, st>>>(a);
   } else {
     if (a.key_valid)
-      dense_split_kernel<T, DH, true><<<(unsigned)small, 256, 0, st>>>(a);
+      dense_split_kernel<T, DH, true><<<groups, 256, 0, st>>>(a);
     else
-      dense_split_kernel<T, DH, false><<<(unsigned)small, 256, 0, st>>>(a);
+      dense_split_kernel<T, DH, false><<<groups, 256, 0, st>>>(a);
   }
   return check_launch("mllm_dense_attention");
 }
@@ -1029,6 +1040,18 @@ int launch_f32(const DenseArgs& a, hipStream_t st) {
 }  // namespace
 }  // namespace mllm
 
+extern "C" int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t q_len) {
+  using namespace mllm;
+  if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || q_len <= 0) return 0;
+  DenseArgs a{};
+  a.B = batch;
+  a.H = num_heads;
+  a.Hkv = num_kv_heads;
+  a.Tq = q_len;
+  a.G = mfma_pack(num_heads / num_kv_heads);
+  return mfma_rows(a);
+}
+
 extern "C" int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb,
                                     int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st,
                                     const uint8_t* key_valid, int64_t kv_sb, int64_t kv_st, int32_t batch,
@@ -1046,10 +1069,9 @@ extern "C" int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, i
   if (batch == 0 || q_len == 0 || num_heads == 0) return MLLM_OK;
   MLLM_REQUIRE(q && k && v && out, MLLM_ERR_INVALID, "mllm_dense_attention: null pointer");
   const int group = num_heads / num_kv_heads;
-  const int pack = 32 % group == 0 ? group : 1;  // query heads per workgroup row of an MFMA kernel
   DenseArgs a{(const char*)q, (const char*)k, (const char*)v, key_valid, (char*)out, q_sb, q_sh, q_st, k_sb, k_sh,
               k_st, v_sb, v_sh, v_st, o_sb, o_sh, o_st, kv_sb, kv_st, batch, num_heads, num_kv_heads, q_len,
-              kv_len, head_dim, pack, softmax_scale};
+              kv_len, head_dim, mfma_pack(group), softmax_scale};
   dim3 grid(q_len, num_heads, batch);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // (more workgroups than a launch takes: dense_kernel, whose grid has the heads and the batch along y and z)

@@ -64,6 +64,7 @@ SIGNATURES = {
     "mllm_dense_attention": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64,
                                             _i64, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _p, _i64, _i64, _i64,
                                             _p]),
+    "mllm_dense_rows": (ctypes.c_int, [_i32, _i32, _i32, _i32]),
     "mllm_rms_norm": (ctypes.c_int, [_p, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
     "mllm_silu_mul": (ctypes.c_int, [_p, _p, _i64, _i32, _p, _p]),
     "mllm_linear_partial": (ctypes.c_int, [_p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i32, _p, _i32, _p]),

@@ -1,4 +1,7 @@
-"""Which calls keep torch's expressions instead of the decoder layer's kernels, as far as that shows without a GPU."""
+"""Which calls keep torch's expressions instead of the decoder layer's kernels, and the rules that size the kernels' launches,
+as far as they show without a GPU."""
+
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
@@ -66,5 +69,16 @@ def test_more_rows_than_a_launch_takes(monkeypatch):
                        ("mllm_sum_partials", (p, 1, 1 << 24, 2048, None, 2, p, None)),
                        ("mllm_sum_partials_norm", (p, 1, p, p, 1 << 24, 8, 1e-5, 2, p, p, None)),
                        ("mllm_rope_table", (p, 1 << 26, p, 64, 2, p, p, None))):
-        with pytest.raises(ValueError, match="fewer than|too many"):
-            call(name, *args)
+        with ThreadPoolExecutor(1) as own, pytest.raises(ValueError, match="fewer than|too many"):
+            own.submit(call, name, *args).result()  # the last error is kept per thread: other tests' stays empty
+
+
+def test_dense_workgroup_rows():
+    # (batch, heads, KV heads, queries): 128 rows only where a head's queries need more than one workgroup of 32
+    from minillm import _native
+
+    rows = _native.lib().fn("mllm_dense_rows")
+    for shape, expected in [((1, 32, 8, 512), 32), ((2, 32, 8, 777), 128), ((4, 32, 8, 777), 128), ((64, 32, 8, 1), 32),
+                            ((64, 32, 8, 8), 32), ((64, 32, 8, 9), 128), ((128, 32, 8, 8), 32), ((16, 32, 32, 32), 32),
+                            ((16, 32, 32, 33), 128), ((12, 32, 32, 33), 128), ((11, 32, 32, 33), 32), ((1, 32, 8, 0), 0)]:
+        assert rows(*shape) == expected, shape
