@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define MLLM_ABI_VERSION 4
+#define MLLM_ABI_VERSION 5
 
 #define MLLM_OK 0
 #define MLLM_ERR_INVALID (-1)
@@ -304,8 +304,8 @@ int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st
                          int32_t dtype, void* out, int64_t o_sb, int64_t o_sh, int64_t o_st, void* stream);
 
 /* Query rows (tokens x query heads that share a KV head) per workgroup mllm_dense_attention takes for a bf16 or fp16 call
- * of this shape on its MFMA kernels: 128 or 32 (0: no such call). */
-int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t q_len);
+ * of this shape on its MFMA kernels on `num_cus` compute units (0: the current device's): 128 or 32 (0: no such call). */
+int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t q_len, int32_t num_cus);
 
 /*
  * RMSNorm of `rows` contiguous rows of `dim` elements (reference src/minillm/model/llama.py:37-49):
@@ -331,14 +331,15 @@ int mllm_rope_table(const int64_t* positions, int64_t n, const float* inv_freq, 
  * as torch.nn.Linear holds them, m <= 64, k a multiple of 256, n multiples of 16, BF16 or F16, fp32 sums, 16-byte
  * aligned pointers.  A row's result depends neither on the other rows nor on m.
  *
- * mllm_linear_ksplit: the number of parts of K that fills the chip for these weights (>= 1).
+ * mllm_linear_ksplit: the number of parts of K that fills `num_cus` compute units (0: the current device's) with these
+ * weights (>= 1).
  * mllm_linear_partial: up to three weights that share x (w1, w2 with n1 = n2 = 0 when absent), K cut into `ksplit`
  * parts: part[ksplit][m][n0 + n1 + n2] fp32, whose sum over the parts is x . w^T.
  * mllm_sum_partials: out [rows, dim] = T(residual + sum of the parts) (residual may be NULL).
  * mllm_sum_partials_norm: sum = T(residual + sum of the parts) and out = its RMSNorm (mllm_rms_norm).
  * mllm_linear_swiglu: out [m, n] = T(silu(x . gate^T) * (x . up^T)).
  */
-int mllm_linear_ksplit(int64_t k, int64_t n0, int64_t n1, int64_t n2);
+int mllm_linear_ksplit(int64_t k, int64_t n0, int64_t n1, int64_t n2, int32_t num_cus);
 int mllm_linear_partial(const void* x, int64_t m, int64_t k, const void* w0, int64_t n0, const void* w1, int64_t n1,
                         const void* w2, int64_t n2, int32_t ksplit, float* part, int32_t dtype, void* stream);
 int mllm_sum_partials(const float* part, int32_t ksplit, int64_t rows, int64_t dim, const void* residual,

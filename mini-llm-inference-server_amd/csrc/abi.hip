@@ -1,4 +1,6 @@
 // Error reporting and version of the C ABI (include/minillm_hip.h).
+#include <atomic>
+
 #include "common.h"
 
 namespace mllm {
@@ -16,6 +18,21 @@ int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MLLM_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
   return MLLM_OK;
+}
+
+int device_cus() {
+  static std::atomic<int> known[64];  // per device, read once (0: not yet)
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
+    cus = known[dev].load(std::memory_order_relaxed);
+    if (cus) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) {
+      known[dev].store(cus, std::memory_order_relaxed);
+      return cus;
+    }
+  }
+  (void)hipGetLastError();  // the failed query is not the next launch's error
+  return 256;
 }
 
 }  // namespace mllm

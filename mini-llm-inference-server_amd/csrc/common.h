@@ -17,6 +17,9 @@ void set_error(const std::string& msg);
 int fail(int code, const std::string& msg);
 // Turns the last launch error (or a HIP status) into MLLM_ERR_HIP with its text.
 int check_launch(const char* what);
+// Compute units of the current device (256, the full chip's, where there is none): what "fills the chip" means in the
+// rules that size a launch.
+int device_cus();
 
 #define MLLM_REQUIRE(cond, code, msg)        \
   do {                                       \

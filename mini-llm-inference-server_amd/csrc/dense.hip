@@ -988,17 +988,16 @@ int64_t items(const DenseArgs& a, int rows) {
   return (int64_t)((a.Tq + tokens - 1) / tokens) * a.B * (a.H / a.G);
 }
 
-// Rows per workgroup of the 16-bit kernels: 128 from 1.5 workgroups per CU of the full chip (256) on, if they are fewer than those of 32, else 32.
-// Measured (bf16, 32 query and 8 KV heads, Dh 128; 128 rows against 32, us): 128 workgroups of 128 rows (one sequence of
+// Rows per workgroup of the 16-bit kernels: 128 from 1.5 workgroups per CU on, if they are fewer than those of 32, else 32.
+// Measured (256 CUs, bf16, 32 query and 8 KV heads, Dh 128; 128 rows against 32, us): 128 workgroups of 128 rows (one sequence of
 // 512 tokens) 23.4 / 12.5, 256 (one of 1,024) 41.0 / 29.8, 400 (two of 777) 39.0 / 38.4, 384 (four of 384) 21.7 / 26.3,
 // 512 (four of 512) 28.2 / 38.6, 800 (four of 777) 49.4 / 68.8: a workgroup of 32 rows reads four times the K and V per
 // row.  Where one workgroup of either size holds all of a head's queries, the 128-row one leaves wavefronts without a row,
 // and one that has some walks all the keys: 1 or 8 queries on 1,024 keys, 64 sequences 47.4 / 43.0 and 48.2 / 43.8, 12 queries
 // (two workgroups of 32 rows) 56.2 / 82.9.
-constexpr int64_t kLargeMin = 384;
-int mfma_rows(const DenseArgs& a) {
+int mfma_rows(const DenseArgs& a, int cus) {
   const int64_t large = items(a, 128);
-  return large >= kLargeMin && large < items(a, 32) ? 128 : 32;
+  return 2 * large >= 3 * (int64_t)cus && large < items(a, 32) ? 128 : 32;
 }
 
 // Query heads of one KV head that share a row of the 16-bit kernels' workgroups.
@@ -1006,7 +1005,7 @@ int mfma_pack(int group) { return 32 % group == 0 ? group : 1; }
 
 template <typename T, int DH>
 int launch_mfma(const DenseArgs& a, hipStream_t st) {
-  const int rows = mfma_rows(a);
+  const int rows = mfma_rows(a, device_cus());
   const unsigned groups = (unsigned)items(a, rows);
   if (rows == 128) {
     if (a.key_valid)
@@ -1040,7 +1039,8 @@ int launch_f32(const DenseArgs& a, hipStream_t st) {
 }  // namespace
 }  // namespace mllm
 
-extern "C" int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t q_len) {
+extern "C" int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t q_len,
+                               int32_t num_cus) {
   using namespace mllm;
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || q_len <= 0) return 0;
   DenseArgs a{};
@@ -1049,7 +1049,7 @@ extern "C" int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_
   a.Hkv = num_kv_heads;
   a.Tq = q_len;
   a.G = mfma_pack(num_heads / num_kv_heads);
-  return mfma_rows(a);
+  return mfma_rows(a, num_cus > 0 ? num_cus : device_cus());
 }
 
 extern "C" int mllm_dense_attention(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb,

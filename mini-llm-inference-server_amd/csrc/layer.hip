@@ -92,9 +92,9 @@ struct LayerScratch {
 
 LayerScratch layer_scratch(int64_t m, int64_t hidden, int64_t ffn, int64_t q, int64_t kv) {
   LayerScratch s;
-  s.ks_qkv = mllm_linear_ksplit(hidden, q, kv, kv);
-  s.ks_o = mllm_linear_ksplit(q, hidden, 0, 0);
-  s.ks_down = mllm_linear_ksplit(ffn, hidden, 0, 0);
+  s.ks_qkv = mllm_linear_ksplit(hidden, q, kv, kv, 0);
+  s.ks_o = mllm_linear_ksplit(q, hidden, 0, 0, 0);
+  s.ks_down = mllm_linear_ksplit(ffn, hidden, 0, 0, 0);
   int64_t at = 0;
   auto take = [&](int64_t bytes) {
     const int64_t here = at;

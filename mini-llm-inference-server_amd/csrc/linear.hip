@@ -171,14 +171,14 @@ int check_operands(const char* fn, const void* x, int64_t m, int64_t k, int32_t 
 }  // namespace
 }  // namespace mllm
 
-// Parts of K per output tile: as many as give every CU of the full chip (256) about one workgroup, so that the launch
-// is one round (o of Llama-3.1-8B 9.4 us at 8 parts against 12.5 at 4; q, k and v 13.7 at 5 against 14.3 at 4), at
-// most 8 (each part's sums are written and read again) and none shorter than two chunks.
-extern "C" int mllm_linear_ksplit(int64_t k, int64_t n0, int64_t n1, int64_t n2) {
+// Parts of K per output tile: as many as give every CU about one workgroup, so that the launch is one round (256 CUs: o of
+// Llama-3.1-8B 9.4 us at 8 parts against 12.5 at 4; q, k and v 13.7 at 5 against 14.3 at 4), at most 8 (each part's sums
+// are written and read again) and none shorter than two chunks.
+extern "C" int mllm_linear_ksplit(int64_t k, int64_t n0, int64_t n1, int64_t n2, int32_t num_cus) {
   using namespace mllm;
   int64_t tiles = 0;
   for (const int64_t n : {n0, n1, n2}) tiles += (n + kTileRows - 1) / kTileRows;
-  int64_t ks = tiles > 0 ? 256 / tiles : 1;
+  int64_t ks = tiles > 0 ? (num_cus > 0 ? num_cus : device_cus()) / tiles : 1;
   if (ks > 8) ks = 8;
   if (ks > k / kChunk / 2) ks = k / kChunk / 2;
   return ks < 1 ? 1 : (int)ks;

@@ -16,7 +16,7 @@ LIB_PATH = Path(os.environ.get("MLLM_HIP_LIB", Path(__file__).resolve().parent /
 
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_HIP = 0, -1, -2, -3
 DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _p = ctypes.c_void_p
 _i32 = ctypes.c_int32
@@ -64,7 +64,7 @@ SIGNATURES = {
     "mllm_dense_attention": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64,
                                             _i64, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _p, _i64, _i64, _i64,
                                             _p]),
-    "mllm_dense_rows": (ctypes.c_int, [_i32, _i32, _i32, _i32]),
+    "mllm_dense_rows": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i32]),
     "mllm_rms_norm": (ctypes.c_int, [_p, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
     "mllm_silu_mul": (ctypes.c_int, [_p, _p, _i64, _i32, _p, _p]),
     "mllm_linear_partial": (ctypes.c_int, [_p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i32, _p, _i32, _p]),
@@ -72,7 +72,7 @@ SIGNATURES = {
     "mllm_sum_partials_norm": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _i64, _f32, _i32, _p, _p, _p]),
     "mllm_linear_swiglu": (ctypes.c_int, [_p, _i64, _i64, _p, _p, _i64, _i32, _p, _p]),
     "mllm_rope_table": (ctypes.c_int, [_p, _i64, _p, _i32, _i32, _p, _p, _p]),
-    "mllm_linear_ksplit": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
+    "mllm_linear_ksplit": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i32]),
     "mllm_decoder_layer_scratch_bytes": (ctypes.c_int64, [_i64, _i64, _i64, _i32, _i32, _i32]),
     "mllm_decoder_layer": (ctypes.c_int, [_p, _p, _i64, _p, _f32, _p, _p, _p, _p, _p, _f32, _p, _p, _p, _i64, _p, _p, _i64,
                                           _p, _p, _f32, _f32, _p, _i64, _p, _p]),

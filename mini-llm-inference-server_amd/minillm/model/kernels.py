@@ -146,7 +146,7 @@ def _partial(x: torch.Tensor, weights) -> tuple[torch.Tensor, int, int]:
     k = x.shape[-1]
     m = x.numel() // k
     rows = [w.shape[0] for w in weights]
-    ks = _native.lib().fn("mllm_linear_ksplit")(k, *rows, *(0,) * (3 - len(rows)))
+    ks = _native.lib().fn("mllm_linear_ksplit")(k, *rows, *(0,) * (4 - len(rows)))
     part = torch.empty(ks * m * sum(rows), dtype=torch.float32, device=x.device)
     args = []
     for w in weights:

@@ -81,4 +81,16 @@ def test_dense_workgroup_rows():
     for shape, expected in [((1, 32, 8, 512), 32), ((2, 32, 8, 777), 128), ((4, 32, 8, 777), 128), ((64, 32, 8, 1), 32),
                             ((64, 32, 8, 8), 32), ((64, 32, 8, 9), 128), ((128, 32, 8, 8), 32), ((16, 32, 32, 32), 32),
                             ((16, 32, 32, 33), 128), ((12, 32, 32, 33), 128), ((11, 32, 32, 33), 32), ((1, 32, 8, 0), 0)]:
-        assert rows(*shape) == expected, shape
+        assert rows(*shape, 256) == expected, shape
+
+
+def test_launch_rules_follow_the_cu_count():
+    from minillm import _native
+
+    rows, parts = _native.lib().fn("mllm_dense_rows"), _native.lib().fn("mllm_linear_ksplit")
+    # one sequence of 512 tokens: 128 workgroups of 128 rows, 1.5 per CU up to 85 CUs
+    assert [rows(1, 32, 8, 512, cus) for cus in (256, 86, 85, 32)] == [32, 32, 128, 128]
+    # q, k and v of Llama-3.1-8B: 48 tiles; o: 32; never below 1 part, nor parts of less than two chunks of 256
+    assert [parts(4096, 4096, 1024, 1024, cus) for cus in (256, 128, 64, 32)] == [5, 2, 1, 1]
+    assert [parts(4096, 4096, 0, 0, cus) for cus in (256, 128, 64, 32)] == [8, 4, 2, 1]
+    assert parts(512, 16, 0, 0, 256) == 1 and parts(1024, 16, 0, 0, 256) == 2
