@@ -46,7 +46,7 @@ def test_edges(hip, dtype, b, h, hkv, tq, tk, dh):
     _compare(_run(q, k, v), torch_ref.prefill(q.double(), k.double(), v.double()), dtype)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("b,h,hkv,tq,tk", [(3, 8, 2, 70, 200), (4, 64, 64, 300, 333), (2, 2, 1, 3, 4700)])
 def test_key_valid(hip, dtype, dh, b, h, hkv, tq, tk):
@@ -59,7 +59,23 @@ def test_key_valid(hip, dtype, dh, b, h, hkv, tq, tk):
     _compare(_run(q, k, v, valid), torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid), dtype)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mask_windows_of_128_row_workgroups(hip, dtype):
+    # 384 workgroups of 128 query rows on 4,700 keys, whose mask takes two windows of 4,096: a row whose first real key
+    # lies in the second, one without a real key, one whose keys run through both
+    from minillm import _native
+
+    b, h, tq, tk = 3, 64, 256, 4700
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _native.lib().fn("mllm_dense_rows")(b, h, 1, tq, 0) == 128
+    q, k, v = _inputs(b, h, 1, tq, tk, 64, dtype, seed=8)
+    valid = torch.rand(b, tk, generator=torch.Generator().manual_seed(9)) < 0.7
+    valid[0, :4500] = False
+    valid[1] = False
+    _compare(_run(q, k, v, valid), torch_ref.prefill(q.double(), k.double(), v.double(), key_valid=valid), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("h", [2, 128])
 def test_values_behind_masked_keys_do_not_leak(hip, dtype, h):
     # key 40 is not finite: queries before it and (masked) all queries of batch row 1 never see it
