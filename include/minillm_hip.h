@@ -311,14 +311,14 @@ int mllm_dense_rows(int32_t batch, int32_t num_heads, int32_t num_kv_heads, int3
  * RMSNorm of `rows` contiguous rows of `dim` elements (reference src/minillm/model/llama.py:37-49):
  * out = weight * T(x * rsqrt(mean(x^2) + eps)), fp32 arithmetic, T the 16-bit `dtype` (BF16 or F16).  With
  * `residual` and `sum` (both or neither), x is first replaced by T(x + residual), which is written to `sum`
- * (reference llama.py:125, the sum before the second norm).  dim a multiple of 8, pointers 16-byte aligned; `out`
- * and `sum` overlap no input.
+ * (reference llama.py:125, the sum before the second norm).  dim a multiple of 8, fewer than 2^24 rows, pointers 16-byte
+ * aligned; `out` and `sum` overlap no input.
  */
 int mllm_rms_norm(const void* x, const void* residual, const void* weight, int64_t rows, int64_t dim, float eps,
                   int32_t dtype, void* sum, void* out, void* stream);
 
 /* out = T(silu(gate) * up) over n contiguous elements, fp32 arithmetic (reference llama.py:117-120); n a multiple of
- * 8, pointers 16-byte aligned. */
+ * 8 and less than 2^35 - 2047, pointers 16-byte aligned. */
 int mllm_silu_mul(const void* gate, const void* up, int64_t n, int32_t dtype, void* out, void* stream);
 
 /* Rotary tables (reference src/minillm/model/llama.py:51-56): cos / sin [n, 2 half] = T(cos / sin(float(positions[t]) *

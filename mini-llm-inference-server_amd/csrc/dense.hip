@@ -3,7 +3,7 @@
 //
 // q [B, H, Tq, Dh], k/v [B, Hkv, Tk, Dh] with arbitrary element strides; query i sits at position
 // Tk - Tq + i and sees keys 0 .. Tk - Tq + i; with key_valid [B, Tk] it sees only real keys among them,
-// and a query that has none sees its own position.  Three kernels:
+// and a query that has none sees its own position.  Four kernels:
 //   dense_mfma_kernel   bf16 / fp16, Dh 64 or 128, 16-byte aligned rows: workgroups of 128 query rows whose
 //                       four wavefronts share each 64-key K/V tile through LDS (many rows);
 //   dense_split_kernel  the same operands: workgroups of 32 query rows whose four wavefronts share the keys

@@ -234,8 +234,9 @@ class DeviceBlockTables:
 
 def _staging(n: int) -> torch.Tensor:
     """Pinned int32 memory for one upload.  A copy out of pageable memory returns only when the stream has reached it,
-    so each step waited for the one before (decode steps of 32 rows 623 against 511 us); out of pinned memory it is
-    enqueued, and torch's host allocator gives the block to a later step only once the copy has run."""
+    so each step waited for the one before (decode steps of 32 rows enqueued one behind the other: 623 against 511 us; an
+    engine step whose sampler reads the tokens finds the stream idle, and gains only the wait for its own copy); out of
+    pinned memory it is enqueued, and torch's host allocator gives the block to a later step only once the copy has run."""
     return torch.empty(n, dtype=torch.int32, pin_memory=True)
 
 

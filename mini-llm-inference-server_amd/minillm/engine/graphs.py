@@ -15,8 +15,8 @@ The graph is captured with fixed sizes.  A row may hold up to ceil(max_model_len
 the decode plan's capacity of a B-row bucket covers every step of up to the fewer pages of B rows at that
 length and the whole pool plus one page per row (without prefix sharing, a step's pages never exceed the
 pool), each at the split size the host heuristic picks for its page count.  Each replay stages the split size an eager step of the same rows would
-use (mllm_plan_dev reads it on the device), so a replayed step runs the same decode work as the eager
-one; a step whose plan at that size exceeds the bucket's capacity (rows sharing prefix pages can) is
+use (mllm_plan_dev reads it on the device), so a replayed step that fills its bucket runs the same decode
+work as the eager one (padding rows add a page each, which moves the cuts between bins); a step whose plan at that size exceeds the bucket's capacity (rows sharing prefix pages can) is
 not replayed but run eagerly (`fits`).  Every replay fills the plan buffers with -1 before planning,
 and the decode and merge launches cover the capacity: workgroups past the step's own bins and merges
 exit at once.  Rows past the step's own are padding (see StaticDecodeMetadata).  All buckets share one decode
@@ -122,7 +122,7 @@ class DecodeGraphs:
 
     def _split(self, pages: int) -> int:
         """The split size an eager step over `pages` decode pages uses with this pool.  A replay cuts the same
-        bins, so its output is the eager step's bit for bit; its decode launch, planned at the smallest
+        bins where the step fills its bucket, so its attention is the eager step's bit for bit; its decode launch, planned at the smallest
         split, runs 4-wavefront workgroups over them (the launch shape does not change a wavefront's
         arithmetic)."""
         return pages_per_split(pages, self.num_kv_heads, self.num_heads, self.cache.quantized,
